@@ -520,9 +520,8 @@ int mzk_sparse_mqa_advance(const void* q, int64_t B, int64_t S, int H, int D, in
  * the list is also written to idx_out [B, idx_out_stride] int32.  With advance != 0 the
  * positions then advance as in mzk_sparse_mqa_advance.  In one launch for the FP8 latent
  * rows (fmt 1, D 576, nope 512) with G <= 8192 and topk <= 2048, both multiples of 4,
- * score_stride and idx_out_stride multiples of 4, scores / idx_out 16-byte aligned, and
- * splits of at most 1024 - 96 entries ((window + dense_cap + topk) / nsplit, the decode
- * kernel's entry tables); otherwise mzk_topk_rows and then the attention, same results.
+ * score_stride and idx_out_stride multiples of 4 and scores / idx_out 16-byte aligned;
+ * otherwise mzk_topk_rows and then the attention, same results.
  * out and lse NULL (nsplit > 1, advance 0): the split partials only, as mzk_sparse_mqa.  Other arguments
  * as mzk_sparse_mqa_rope (rope_cos / rope_sin may be NULL).  No counterpart in the
  * reference as one call: it is the reference's index_scores.topk followed by its sparse

@@ -16,19 +16,16 @@
 // Entry formats: bf16 [D] rows, or the 656 B FP8-b128 latent entry (512 e4m3 + 4 fp32
 // scales + 64 bf16 rope), dequantized on load.
 //
-// Tiling (MI355X): one workgroup = one (row, split, group of <= 64 heads); HG x DS waves,
-// HG = head groups of 32 (the MFMA N axis), DS = number of D-parts (2 when D > 256, so a
-// wave's q fragments + O^T accumulators fit one SIMD's registers).  Per 32-entry tile:
+// Two kernels over the same plan of a row (RowPlan): attention_latent.h for D = 576, and here
+// for D <= 256 one wave per 32 heads over the whole of D.  Per 32-entry tile of the latter:
 //   1. the tile (fetched from HBM into registers while the previous tile computed) is
 //      dequantized to bf16 into LDS, Kt[entry][d];
-//   2. S^T[32 entries x 32 heads] = Kt . Q^T on v_mfma_f32_32x32x16_bf16, each wave over its
-//      D-part, partial sums exchanged through LDS (fixed order: part 0 + part 1);
+//   2. S^T[32 entries x 32 heads] = Kt . Q^T on v_mfma_f32_32x32x16_bf16;
 //   3. online softmax in the exp2 domain, lane-local per head (lane l holds head l%32);
-//   4. O^T[d x 32 heads] += V^T . P^T on MFMA, each wave owning its D-part of O: P^T stays
-//      in the registers the S^T result left it in, and the V^T operand is gathered from
-//      Kt columns in the matching entry order.
-// The workgroup writes either the final bf16 output + lse (one split) or fp32 partials
-// (unnormalized O, running max m, sum l) that mzk combine kernel merges with the sink.
+//   4. O^T[d x 32 heads] += V^T . P^T on MFMA: P^T stays in the registers the S^T result left
+//      it in, and the V^T operand is gathered from Kt columns in the matching entry order.
+// A workgroup writes either the final bf16 output + lse (one split) or its split's own
+// normalized output in bf16 and (m, l), which the combine kernel merges with the sink.
 #include <type_traits>
 
 #include <mutex>
@@ -124,14 +121,7 @@ struct Layout {
 // Entry held by register j of lane l in a 32x32 MFMA result: 8*(j/4) + 4*(l/32) + j%4.
 __device__ __forceinline__ int c_entry(int j, int lane) { return 8 * (j >> 2) + 4 * (lane >> 5) + (j & 3); }
 
-// Workgroup barrier that waits only for this wave's LDS operations (not for vector
-// memory: the next tile's loads stay in flight across it).  The "memory" clobber keeps
-// the compiler from moving memory accesses across.
-__device__ __forceinline__ void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" : : : "memory"); }
-
-constexpr int kIdxCap = 4096;       // sparse indices of one split staged in LDS (D <= 256 kernel)
-constexpr int kSplitIdxCap = 1024;  // the same for the D-split kernel (its LDS holds three tiles)
-constexpr int kAllTabCap = 1024;    // D-split kernel: splits of at most this many entries keep every tile's table
+constexpr int kIdxCap = 4096;  // the most entries of one split (staged indices, entry tables in LDS)
 
 typedef const uint8_t __attribute__((address_space(1)))* gptr_t;  // global (not flat) loads
 typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
@@ -185,8 +175,8 @@ __device__ __forceinline__ void store_piece(uint8_t* krow, const Piece& r, int q
 
 // One (row, split, head group)'s share of the row's virtual entry list
 // [window nw | dense nd | sparse ns], the entry tables of its tiles, and the register
-// prefetch of a tile.  Shared by both kernels.
-template <int FMT, int D, int NOPE, int NT, int NSLOT = 2>
+// prefetch of a tile.  The latent kernel shares its plan and list, and has tables of its own.
+template <int FMT, int D, int NOPE, int NT>
 struct RowPlan {
   using L = Layout<FMT, D, NOPE>;
   static constexpr int TPE = NT / kTile;                          // threads per entry
@@ -199,9 +189,8 @@ struct RowPlan {
   const uint8_t* win_b;
   const uint8_t* dense_b;
   const uint8_t* main_b;
-  const uint8_t** tab_ptr;   // [NSLOT][kTile] in LDS: tile t uses slot t & slot_mask
-  uint32_t* tab_mask;        // [NSLOT] in LDS
-  uint32_t slot_mask = NSLOT - 1;  // all the split's tables at once (build_all_tables): ~0
+  const uint8_t** tab_ptr;   // [2][kTile] in LDS: tile t uses slot t & 1
+  uint32_t* tab_mask;        // [2] in LDS
   // typed address spaces: a generic pointer would make these FLAT loads, which count
   // against the LDS wait counter too and force every later LDS wait to drain completely
   const __attribute__((address_space(3))) int32_t* sidx;     // this split's sparse indices (the first sidx_cap), in LDS
@@ -209,7 +198,7 @@ struct RowPlan {
   int sidx_cap;
 
   // Workgroup -> (row, split, head group).  Workgroups are dealt to the 8 XCDs round-robin
-  // (workgroup i runs on XCD i % 8).  ROW_XCD (the decode kernel instance) with rows a
+  // (workgroup i runs on XCD i % 8).  ROW_XCD (the latent kernel) with rows a
   // multiple of 8: every workgroup of row r runs on XCD r % 8: the head groups of a (row, split), which read the same entries, and
   // the splits, which read the same q, share an L2, and so does the merge launch, which maps
   // its workgroups the same way and finds the row's partials there.  Otherwise the head
@@ -221,9 +210,7 @@ struct RowPlan {
     plan(p, p.positions[row]);
   }
 
-  // The workgroup's (row, split, head group); no memory access.  (ROW_XCD is a template
-  // argument so that the other kernel instances compile without its branch: their code,
-  // the prefill's long tile loops included, stays as it was.)
+  // The workgroup's (row, split, head group); no memory access.
   template <bool ROW_XCD = false>
   __device__ void locate(const AttnParams& p, int heads_per_wg) {
     const uint32_t nhg = static_cast<uint32_t>((p.H + heads_per_wg - 1) / heads_per_wg);
@@ -330,70 +317,66 @@ struct RowPlan {
     sidx_cap = cap;
   }
 
-  // Request the row's first 4*NT sparse indices, one 16-byte load per thread, before the
-  // row's position (which fixes this split's slice) is known, so the two loads overlap.
-  // Returns false (and loads nothing) unless the whole list fits and its row is 16-byte
-  // aligned; then stage_indices reads it after the position.
-  __device__ bool prefetch_indices(const AttnParams& p, int tid, v4i& pre) {
-    idx_row = p.idx ? (const __attribute__((address_space(1))) int32_t*)(p.idx + row * p.idx_row_stride) : nullptr;
-    const bool ok = idx_row != nullptr && p.topk > 0 && p.topk <= 4 * NT && (p.topk & 3) == 0 &&
-                    (reinterpret_cast<uintptr_t>(idx_row) & 15u) == 0;
-    // branch-free: every thread loads from a valid address (the query, 16-byte aligned, when
-    // the list is not used), so the compiler's in-order wait counts stay exact
-    const int at = 4 * tid < p.topk ? 4 * tid : p.topk - 4;
-    const __attribute__((address_space(1))) v4i* src =
-        ok ? reinterpret_cast<const __attribute__((address_space(1))) v4i*>(idx_row + at)
-           : (const __attribute__((address_space(1))) v4i*)(p.q);
-    pre = *src;
-    if (!ok || 4 * tid >= p.topk) pre = v4i{-1, -1, -1, -1};
+  // For the latent kernel: request the row's first 8 * NT sparse indices, two 16-byte loads per
+  // thread (list positions 4 tid + 4 NT r), before the row's position (which fixes this split's
+  // slice) is known, so the two overlap.  Returns false unless the whole list fits and its row
+  // is 16-byte aligned; then the table reads the list from memory.
+  __device__ bool prefetch_list(const AttnParams& p, int tid, v4i (&pre)[2]) const {
+    const int32_t* ir = p.idx ? p.idx + row * p.idx_row_stride : nullptr;
+    const bool ok = ir != nullptr && p.topk > 0 && p.topk <= 8 * NT && (p.topk & 3) == 0 &&
+                    (reinterpret_cast<uintptr_t>(ir) & 15u) == 0;
+#pragma unroll
+    for (int r = 0; r < 2; ++r) {
+      // branch-free: every thread loads from a valid address (the query when the list is not used)
+      const int o = 4 * tid + 4 * NT * r;
+      const v4i* src = ok ? reinterpret_cast<const v4i*>(ir + (o < p.topk ? o : p.topk - 4))
+                          : reinterpret_cast<const v4i*>(p.q);
+      pre[r] = *src;
+      if (!ok || o >= p.topk) pre[r] = v4i{-1, -1, -1, -1};
+    }
     return ok;
   }
-
-  // stage_indices from the prefetched list (prefetch_indices returned true): the thread
-  // holding list positions 4tid..4tid+3 writes those inside the slice.
-  __device__ void stage_prefetched(int32_t* sidx_lds, int cap, int tid, const v4i& pre) {
-    const int sp_end = v_end > nwd ? v_end - nwd : 0;
-    const int lim = sp_end < sp_begin + cap ? sp_end : sp_begin + cap;
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const int s = 4 * tid + j;
-      if (s >= sp_begin && s < lim) sidx_lds[s - sp_begin] = pre[j];
-    }
-    sidx = (const __attribute__((address_space(3))) int32_t*)(sidx_lds);
-    sidx_cap = cap;
-  }
-
-  // With the whole list prefetched (prefetch_indices returned true): the number of its
-  // leading valid indices (0 <= g < G) when every valid index precedes every invalid one --
-  // the form the top-k launch writes (ascending picks, then -1) -- else topk.  Walking only
-  // that prefix skips tiles that would be all masked.  `wred` is 2 * (NT / 64) ints of LDS;
-  // two workgroup barriers.
-  __device__ int valid_prefix(const AttnParams& p, int tid, const v4i& pre, int* wred) const {
+  // With the whole list prefetched: the number of its leading valid indices (0 <= g < G) when
+  // every valid index precedes every invalid one -- the form the top-k launch writes
+  // (ascending picks, then -1) -- else topk.  Walking only that prefix skips tiles that would
+  // be all masked.  `wred` is 2 * (NT / 64) ints of LDS; one workgroup barrier.
+  __device__ int valid_prefix_list(const AttnParams& p, int tid, const v4i (&pre)[2], int* wred) const {
     constexpr int NW = NT / 64;
     const int lane = tid & 63, wave = tid >> 6;
     const int64_t glim = p.G;
-    auto valid = [&](int j) { return 4 * tid + j < p.topk && pre[j] >= 0 && pre[j] < glim; };
-    int c = 0;
+    int c = 0, last = -1;  // valid indices, and the list position of the last one
 #pragma unroll
-    for (int j = 0; j < 4; ++j) c += valid(j);
-    int wc = c;
+    for (int r = 0; r < 2; ++r)
 #pragma unroll
-    for (int m = 32; m >= 1; m >>= 1) wc += __shfl_xor(wc, m, 64);
-    if (lane == 0) wred[wave] = wc;
+      for (int j = 0; j < 4; ++j) {
+        const int at = 4 * tid + 4 * NT * r + j;
+        if (at < p.topk && pre[r][j] >= 0 && pre[r][j] < glim) {
+          ++c;
+          last = at;
+        }
+      }
+#pragma unroll
+    for (int m = 32; m >= 1; m >>= 1) {
+      c += __shfl_xor(c, m, 64);
+      last = max(last, __shfl_xor(last, m, 64));
+    }
+    if (lane == 0) {
+      wred[wave] = c;
+      wred[NW + wave] = last;
+    }
     __syncthreads();
-    int n = 0;
+    int n = 0, end = -1;
 #pragma unroll
-    for (int w = 0; w < NW; ++w) n += wred[w];
-    bool bad = false;
+    for (int w = 0; w < NW; ++w) {
+      n += wred[w];
+      end = max(end, wred[NW + w]);
+    }
+    return end + 1 == n ? n : p.topk;
+  }
+  // The prefetched list in LDS, 16-byte aligned, 8 * NT entries.
+  __device__ void stage_list(int32_t* list, int tid, const v4i (&pre)[2]) const {
 #pragma unroll
-    for (int j = 0; j < 4; ++j) bad |= valid(j) && 4 * tid + j >= n;
-    const uint64_t bb = __ballot(bad);
-    if (lane == 0) wred[NW + wave] = bb != 0;
-    __syncthreads();
-    int nb = 0;
-#pragma unroll
-    for (int w = 0; w < NW; ++w) nb += wred[NW + w];
-    return nb ? p.topk : n;
+    for (int r = 0; r < 2; ++r) *reinterpret_cast<v4i*>(list + 4 * tid + 4 * NT * r) = pre[r];
   }
 
   // sparse index of list position v (-1 outside the sparse part of this split)
@@ -426,66 +409,17 @@ struct RowPlan {
   __device__ void build_table(const AttnParams& p, int t, int g, int tid) {
     if (tid < kTile) {
       const uint8_t* ptr = entry_ptr(p, t, tid, g);
-      tab_ptr[(t & slot_mask) * kTile + tid] = ptr;
+      tab_ptr[(t & 1) * kTile + tid] = ptr;
       const uint64_t bal = __ballot(ptr != nullptr);
-      if (tid == 0) tab_mask[t & slot_mask] = static_cast<uint32_t>(bal);
+      if (tid == 0) tab_mask[t & 1] = static_cast<uint32_t>(bal);
     }
-  }
-
-  // entry tables of tiles 0..3 at once (after the indices are staged): thread tid < 4*kTile
-  // fills entry tid % kTile of tile tid / kTile, two tiles per wave
-  __device__ void build_first_tables(const AttnParams& p, int tid) {
-    static_assert(NSLOT >= 4 && NT >= 4 * kTile, "four tables in flight");
-    if (tid < 4 * kTile) {
-      const int t = tid / kTile, e = tid % kTile;
-      const uint8_t* ptr = entry_ptr(p, t, e, slot(v_begin + t * kTile + e));
-      tab_ptr[t * kTile + e] = ptr;
-      const uint64_t bal = __ballot(ptr != nullptr);
-      if (e == 0) tab_mask[t] = static_cast<uint32_t>(bal >> (32 * (t & 1)));
-    }
-  }
-
-  // Tables the D-split tile loop reads: tiles 0..3 (its prologue) and up to three past the
-  // last tile (it fetches tile u+3 while at tile u), whose entries are all empty.
-  __device__ int table_tiles() const { return ntiles + 3 > 4 ? ntiles + 3 : 4; }
-
-  // Every entry table the tile loop reads (table_tiles()), at once, when they fit `CAP`
-  // pointers at `all` (which may overlap the staged sparse indices: each thread reads its
-  // indices before a barrier, then writes).  Tile t then uses table t, and the tile loop
-  // builds none.  Entry e = tid + NT * r; a wave's ballot covers tiles 2w' and 2w'+1.
-  // One workgroup barrier; the caller synchronises before the tables are read.
-  template <int CAP>
-  __device__ void build_all_tables(const AttnParams& p, int tid, const uint8_t** all, uint32_t* masks) {
-    static_assert(CAP % NT == 0 && NT % 64 == 0, "whole waves per round");
-    constexpr int R = CAP / NT;
-    const int n = table_tiles() * kTile;  // <= CAP (the caller checks)
-    int g[R];
-#pragma unroll
-    for (int r = 0; r < R; ++r) {
-      const int e = tid + NT * r;
-      g[r] = e < n ? slot(v_begin + e) : -1;
-    }
-    __syncthreads();  // every staged index is read before the tables overwrite them
-#pragma unroll
-    for (int r = 0; r < R; ++r) {
-      const int e = tid + NT * r;
-      const bool in = e < n;
-      const uint8_t* ptr = in ? entry_ptr(p, e / kTile, e % kTile, g[r]) : nullptr;
-      if (in) all[e] = ptr;
-      const uint64_t bal = __ballot(ptr != nullptr);
-      const int lane = tid & 63;
-      if (in && (lane & 31) == 0) masks[e / kTile] = static_cast<uint32_t>(lane ? bal >> 32 : bal);
-    }
-    tab_ptr = all;
-    tab_mask = masks;
-    slot_mask = ~0u;
   }
 
   // The tile's pieces for this thread: entry tid / TPE, pieces (tid % TPE) + TPE*k, so the
   // TPE threads of an entry read TPE consecutive 16-byte pieces per load instruction.
   // Empty slots load zeros.
   __device__ void fetch(int t, int tid, Piece (&raw)[PPT]) const {
-    const gptr_t e = (gptr_t)(tab_ptr[(t & slot_mask) * kTile + tid / TPE]);
+    const gptr_t e = (gptr_t)(tab_ptr[(t & 1) * kTile + tid / TPE]);
 #pragma unroll
     for (int k = 0; k < PPT; ++k) {
       const int q = tid % TPE + TPE * k;
@@ -984,543 +918,7 @@ __global__ void __launch_bounds__(HG * 64) sparse_mqa_kernel(const AttnParams p)
   write_result<D, NOPE, NB>(p, rp.row, rp.b, rp.split, head, half, half == 0, 0, NB, m_run, l_run, acc_o);
 }
 
-// ------------------------------------------------------------------------------------
-// D > 256 (the 512+64 latent): 64 heads per workgroup, each 32-head group split over 4
-// waves by D (8 waves, two per SIMD: one of each group).  A wave holds its D-quarter of q
-// (9 K-steps) and at most 5 O^T blocks; the four partial S^T of a head group are summed
-// through LDS.  The two groups run half a tile apart (ping-pong), so on every SIMD one
-// wave does MFMA work (PV of one tile interleaved with QK of the next, operands read a
-// block ahead) while the other does the softmax, its half of the next tile's
-// dequantization into LDS, and the tile fetches; the schedule is spelled out at the
-// tile loop.  Softmax: the running max is raised lazily to an upper bound of the tile
-// max (the sum of the four partial maxima), so exp2(s - m) <= 2^kLazy always holds; the
-// online softmax is exact for any reference point as long as no significant term
-// underflows, which the pass checks at its end (else an exact pass redoes the split).
-// One barrier per half-tile (one more per half-tile in the exact pass, which exchanges
-// the true tile max).
-// ------------------------------------------------------------------------------------
-template <int FMT, int D, int NOPE>
-struct SplitSmem {
-  static constexpr int HG = 2, DS = 4;
-  static constexpr int KT_PITCH = 2 * D + 16;
-  static constexpr int KT = kTile * KT_PITCH;             // one bf16 tile
-  static constexpr int SX = HG * DS * 4 * 64 * 16;        // [wave][4][64] float4 partial S^T
-  static constexpr int PM = HG * 32 * 2 * DS * 4;         // [2][64 heads] float4: partial maxima / row sums
-  static constexpr int PB = HG * 2 * 64 * 16;             // [hg][2 K-steps][64] P^T
-  static constexpr int PE = HG * 32 * 2 * DS * 4;         // [2][64 heads] float4: true lane maxima
-  static constexpr int NKT = 3;                            // bf16 tiles in flight: PV, QK, dequantized
-  static constexpr int LDS = NKT * KT + SX + PM + PB + PE;
-};
-
-// ALLTAB: the host has checked that every split of the launch keeps all its entry tables
-// (its longest possible split does), so the ring of tables and its index reads (which may
-// go to global memory, and whose waits would then also drain the tile loads in flight) are
-// compiled out.
-// SEL (with ALLTAB): the workgroup selects its row's sparse list itself from the indexer
-// scores (topk_core.h's row selection, 16 scores per thread: G <= 8192, topk <= 2048, both
-// multiples of 4), in the LDS the tiles take later -- every workgroup of the row computes
-// the same list, so no workgroup waits for another and the top-k launch goes away.
-template <int FMT, int D, int NOPE, bool ALLTAB, bool SEL = false>
-__global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2)))
-sparse_mqa_dsplit_kernel(const AttnParams p) {
-  using M = SplitSmem<FMT, D, NOPE>;
-  constexpr int HG = M::HG, DS = M::DS;
-  constexpr int NT = HG * DS * 64;
-  constexpr int KT_PITCH = M::KT_PITCH;
-  constexpr int QST = D / 16 / DS;            // QK K-steps per wave
-  constexpr int NB = D / 32;                  // 32-channel blocks of O
-  constexpr int NDBM = (NB + DS - 1) / DS;    // most O blocks one wave owns
-  // entry tables in flight: t (its mask), t+1 .. t+3 (fetched), t+4 (built this tile)
-  constexpr int NSLOT = 8;
-  using RP = RowPlan<FMT, D, NOPE, NT, NSLOT>;
-  static_assert((D / 16) % DS == 0 && D % 32 == 0, "D must split into 4 parts of 16-channel steps");
-
-  extern __shared__ __align__(16) uint8_t smem[];
-  uint8_t* kt0 = smem;                                                   // 3 x [32][KT_PITCH]
-  float4* sx = reinterpret_cast<float4*>(smem + M::NKT * M::KT);
-  float* pm = reinterpret_cast<float*>(smem + M::NKT * M::KT + M::SX);
-  uint4* pb = reinterpret_cast<uint4*>(smem + M::NKT * M::KT + M::SX + M::PM);
-  float* pe = reinterpret_cast<float*>(smem + M::NKT * M::KT + M::SX + M::PM + M::PB);
-  // one LDS region for the entry tables: the staged sparse indices (first 4 KB) and a ring
-  // of NSLOT tables after them, or -- when the split has at most kAllTabCap entries --
-  // every table of the split over the whole region (built once, before the passes)
-  static_assert(kSplitIdxCap * 4 + NSLOT * kTile * 8 <= kAllTabCap * 8, "ring and indices share the region");
-  __shared__ __align__(16) const uint8_t* tabs[kAllTabCap];
-  __shared__ uint32_t tab_mask[kAllTabCap / kTile];
-  int32_t* sidx = reinterpret_cast<int32_t*>(tabs);
-  const uint8_t** tab_ptr = tabs + kSplitIdxCap / 2;
-  __shared__ int redo;  // set when the fast pass's running max drifted too far above the truth
-
-  const int tid = threadIdx.x;
-  const int lane = tid & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);  // wave-uniform (scalar) branches on the group
-  const int hg = wave / DS;
-  if (tid == 0) redo = 0;  // published by the barrier after the indices are staged
-  const int ds = wave % DS;
-  const int half = lane >> 5;
-  RP rp;
-  rp.tab_ptr = tab_ptr;
-  rp.tab_mask = tab_mask;
-  rp.template locate<ALLTAB>(p, HG * 32);
-  // The row's index list (SEL: its scores), its position and this lane's query fragment are
-  // requested together: one memory round trip at the start instead of three dependent ones.
-  v4i pre;
-  bool pre_ok;
-  constexpr int SKPT = 16;  // SEL: scores per thread
-  static_assert(!SEL || (ALLTAB && SKPT * NT == 8192), "the selecting instance: decode, 8192 scores per row");
-  float4 sc4[SEL ? SKPT / 4 : 1];
-  if constexpr (SEL) {
-    // branch-free: G is a multiple of 4, so a thread's last aligned float4 at or past the
-    // row's end is re-read from G - 4 (and its keys are padding below)
-    const float* srow = p.sel_scores + rp.row * p.sel_stride;
-    const int G4 = static_cast<int>(p.G) - 4;
-#pragma unroll
-    for (int m = 0; m < SKPT / 4; ++m) {
-      const int o = SKPT * tid + 4 * m;
-      sc4[m] = *reinterpret_cast<const float4*>(srow + (o <= G4 ? o : G4));
-    }
-    pre_ok = true;
-  } else {
-    pre_ok = rp.prefetch_indices(p, tid, pre);
-  }
-  const int64_t row_pos = p.positions[rp.row];
-
-  const int hl = hg * 32 + (lane & 31);  // head within the workgroup
-  const int head = rp.hgrp * (HG * 32) + hl;
-  const bool head_ok = head < p.H;
-  const int qc0 = ds * QST * 16;  // first QK channel of this wave
-  // this lane's slot k = 2 ds + half of its head's eight partial maxima / row sums, in a
-  // [2][64 heads] float4 layout: a head's eight values are two conflict-free float4 reads,
-  // and a wave's 64 b32 writes fall on 32 distinct banks (2-way; [64 heads][8] was 8-way)
-  const int pm_slot = (((2 * ds + half) >> 2) * 64 + hl) * 4 + ((2 * ds + half) & 3);
-  v8bf qf[QST];
-  {
-    // branch-free loads (a missing head reads head 0 and is zeroed); uniform row base plus a
-    // 32-bit lane offset (H <= 128) keeps no 64-bit per-lane address alive
-    const uint16_t* qbase = p.q + rp.row * p.H * D;
-    const uint32_t qoff = static_cast<uint32_t>((head_ok ? head : 0) * D + qc0 + half * 8);
-#pragma unroll
-    for (int st = 0; st < QST; ++st) {
-      v4i v = *reinterpret_cast<const v4i*>(qbase + qoff + 16 * st);
-      if (!head_ok) v = v4i{0, 0, 0, 0};
-      qf[st] = __builtin_bit_cast(v8bf, v);
-    }
-  }
-  // RoPE of q: the rope slice is the last RST K-steps of the last D-quarter; every lane
-  // reads the cos / sin of the 4 pairs those steps give it (of the row's first pairs when
-  // no table is given), and the last D-quarter rotates them before its first QK
-  constexpr int RST = (D - NOPE) / 16;
-  static_assert(RST == 0 || ((D - NOPE) % 16 == 0 && D - NOPE <= D / DS), "rope slice inside the last D-quarter");
-  uint2 qrc[RST > 0 ? RST : 1], qrs[RST > 0 ? RST : 1];
-  const bool q_rope = RST > 0 && p.rope_cos != nullptr && ds == DS - 1;
-  if constexpr (RST > 0) {
-    const uint16_t* cb = p.rope_cos ? p.rope_cos : p.q;
-    const uint16_t* sb = p.rope_cos ? p.rope_sin : p.q;
-    const uint32_t roff = static_cast<uint32_t>(rp.row * ((D - NOPE) / 2)) + 4 * half;
-#pragma unroll
-    for (int r = 0; r < RST; ++r) {
-      qrc[r] = *reinterpret_cast<const uint2*>(cb + roff + 8 * r);
-      qrs[r] = *reinterpret_cast<const uint2*>(sb + roff + 8 * r);
-    }
-  }
-  // in-launch merge: the workgroup registers the XCC it runs on with its (row, 64-head
-  // group), after its first loads (an atomic without return: no wait covers it)
-  uint32_t* mrec = nullptr;
-  if constexpr (ALLTAB) {
-    if (p.merge_rec != nullptr) {
-      const uint32_t nhg = static_cast<uint32_t>((p.H + HG * 32 - 1) / (HG * 32));
-      mrec = p.merge_rec + 4 * (static_cast<uint32_t>(rp.row) * nhg + static_cast<uint32_t>(rp.hgrp));
-      if (tid == 0)
-        __hip_atomic_fetch_add(reinterpret_cast<uint64_t*>(mrec), 1ull << (8 * xcc_id()), __ATOMIC_RELAXED,
-                               __HIP_MEMORY_SCOPE_AGENT);
-    }
-  }
-  __shared__ int wred[2 * 8];
-  if constexpr (SEL) {
-    rp.plan_row(p, row_pos);
-    // the row's selection in the tile region of LDS (first written by the tile loop, after
-    // the barriers below): three histograms and the scan scratch
-    int* const h1 = reinterpret_cast<int*>(smem);
-    int* const h2 = h1 + kBins * kSub1;
-    int* const h3 = h2 + kBins;
-    int* const sw = h3 + kBins / 2;
-    static_assert((kBins * kSub1 + kBins + kBins / 2 + 16) * 4 <= M::NKT * M::KT, "selection LDS");
-    const RowSelLds lds{h1, h2, h3, sw, sw + 8, sw + 12};
-    const int G = static_cast<int>(p.G), k = p.topk;
-    const bool search = G > k;
-    if (search) {
-      row_sel_clear<NT>(lds, tid);
-      __syncthreads();
-    }
-    const int i0 = SKPT * tid;
-    uint32_t key[SKPT];
-#pragma unroll
-    for (int m = 0; m < SKPT / 4; ++m) {
-      const float v[4] = {sc4[m].x, sc4[m].y, sc4[m].z, sc4[m].w};
-#pragma unroll
-      for (int c = 0; c < 4; ++c) key[4 * m + c] = order_key(v[c]) & key_mask(i0 + 4 * m + c, G);
-    }
-
-    uint32_t T;
-    int need_eq;
-    row_sel_threshold<SKPT, NT>(key, search, k, lds, T, need_eq);
-    const RowTake tk = row_sel_take<SKPT, NT>(key, T, need_eq, sw);
-    // the list is in the top-k launch's form (ascending picks, then -1) by construction, so
-    // the split is planned over its `written` valid entries directly, and every thread puts
-    // its picks of this split's slice straight into the staged indices (a slice holds at most
-    // kAllTabCap - 96 < kSplitIdxCap entries); the row's first workgroup also writes the list
-    rp.plan_split(p, tk.written);
-    const int sp_end = rp.v_end > rp.nwd ? rp.v_end - rp.nwd : 0;
-    const bool first = p.sel_out != nullptr && rp.split == 0 && rp.hgrp == 0;
-    int32_t* const orow = first ? p.sel_out + rp.row * p.sel_out_stride : nullptr;
-    // a thread's picks take list positions pos .. pos + popcount - 1, ascending with the
-    // thread, so only the threads around this split's slice (and in the row's first
-    // workgroup, every thread) walk them
-    uint32_t sel = tk.sel;
-    if (first || (tk.pos < sp_end && tk.pos + __builtin_popcount(sel) > rp.sp_begin)) {
-      for (int at = tk.pos; sel != 0u; ++at) {
-        const int g = i0 + __builtin_ctz(sel);
-        if (at >= rp.sp_begin && at < sp_end) sidx[at - rp.sp_begin] = g;
-        if (first && at < k) orow[at] = g;
-        sel &= sel - 1u;
-      }
-    }
-    if (first)
-      for (int i = tk.written + tid; i < k; i += NT) orow[i] = -1;
-    rp.sidx = (const __attribute__((address_space(3))) int32_t*)(sidx);
-    rp.sidx_cap = kSplitIdxCap;
-    rp.idx_row = nullptr;  // never read: the slice fits the staged indices
-  } else {
-    rp.plan(p, row_pos, pre_ok ? rp.valid_prefix(p, tid, pre, wred) : -1);
-    if (pre_ok) rp.stage_prefetched(sidx, kSplitIdxCap, tid, pre);
-    else rp.stage_indices(p, sidx, kSplitIdxCap, tid);
-  }
-  __syncthreads();
-  // Splits of at most kAllTabCap entries (every decode configuration) get all their entry
-  // tables here, so the tile loop builds none (a table build costs the building wave an
-  // LDS round trip and the pointer arithmetic on the critical half-step); longer splits
-  // (long prefill rows) build them in a ring as the loop goes.
-  const bool tables_fit = rp.table_tiles() * kTile <= kAllTabCap;
-  const bool all_tables = ALLTAB || tables_fit;
-  if (ALLTAB && !tables_fit) rp.ntiles = 0;  // excluded by the host's check: never read past the tables
-  if (all_tables) rp.template build_all_tables<kAllTabCap>(p, tid, tabs, tab_mask);
-  const int b_lo = ds * NB / DS;
-  const int nb_mine = (ds + 1) * NB / DS - b_lo;
-  const int pv_off = pv_lane_offset<KT_PITCH>(lane, b_lo * 32);
-  // S^T partial over this wave's D-quarter of the tile in `kt`; K fragments are read
-  // three K-steps ahead of their MFMA (a rolling window keeps register pressure low)
-  auto qk = [&](const uint8_t* kt) __attribute__((always_inline)) -> v16f {
-    constexpr int AH = 3;
-    const uint8_t* krow = kt + (lane & 31) * KT_PITCH + 2 * (qc0 + half * 8);
-    uint4 kv[AH];
-#pragma unroll
-    for (int i = 0; i < AH; ++i) kv[i] = *reinterpret_cast<const uint4*>(krow + 32 * i);
-    v16f s = v16f{};
-#pragma unroll
-    for (int st = 0; st < QST; ++st) {
-      const uint4 cur = kv[st % AH];
-      if (st + AH < QST) kv[st % AH] = *reinterpret_cast<const uint4*>(krow + 32 * (st + AH));
-      const v8bf kf = __builtin_bit_cast(v8bf, v4i{(int)cur.x, (int)cur.y, (int)cur.z, (int)cur.w});
-      s = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf, qf[st], s, 0, 0, 0);
-    }
-    return s;
-  };
-  // the partial ([wave][j/4][lane] float4: consecutive lanes at consecutive 16 B,
-  // conflict-free) and its per-head maximum over this lane's 16 entries go to LDS
-  auto publish = [&](const v16f& s) __attribute__((always_inline)) {
-    float mx = s[0];
-#pragma unroll
-    for (int j = 1; j < 16; ++j) mx = fmaxf(mx, s[j]);
-    pm[pm_slot] = mx;
-#pragma unroll
-    for (int j4 = 0; j4 < 4; ++j4)
-      sx[(wave * 4 + j4) * 64 + lane] = float4{s[4 * j4], s[4 * j4 + 1], s[4 * j4 + 2], s[4 * j4 + 3]};
-  };
-
-  // One pass over the split.  The fast pass raises the running max to the partial-maxima
-  // bound, which may exceed the true maximum; it tracks each head's true maximum on the
-  // side and gives up (returns false, writes nothing) if the final running max lies more
-  // than kBoundSlack above it.  Below that every entry that v_exp_f32 flushes to zero
-  // (argument < -126) weighs less than 2^-62 of the largest entry, so the result is exact
-  // to fp32 resolution.  The exact pass (only run after a fast pass gave up) exchanges
-  // the true tile max through LDS with one more barrier per tile.
-  constexpr float kBoundSlack = 64.0f;
-  auto pass = [&](auto exact_tag) -> bool {
-    constexpr bool kExact = decltype(exact_tag)::value;
-    v16f acc_o[NDBM];
-#pragma unroll
-    for (int i = 0; i < NDBM; ++i) acc_o[i] = v16f{};
-    float m_run = -__builtin_huge_valf();  // identical in the 8 lanes x waves of a head
-    float l_run = 0.0f;                    // this lane's share of the head's row sum
-    float m_seen = -__builtin_huge_valf(); // true max of this lane's (unmasked) entries
-
-    // Ping-pong schedule.  The two head groups run half a tile apart, so on every SIMD
-    // (which holds one wave of each group) one wave does MFMA work while the other does
-    // the softmax and the tile traffic.  Half-step 2u (even) and 2u+1 (odd), each opened by
-    // a workgroup barrier:
-    //   even(u): group 0 softmax(u) -> P^T(u); stores its half (entries 16..31) of tile u+1,
-    //            fetches its half of tile u+3, builds the entry table of tile u+4;
-    //            group 1 PV(u-1) + QK(u) -> publishes S^T(u).
-    //   odd(u):  group 0 PV(u) + QK(u+1) -> publishes S^T(u+1);
-    //            group 1 softmax(u) -> P^T(u); stores its half (entries 0..15) of tile
-    //            u+2, fetches its half of tile u+4.
-    // Tile u lives in LDS tile u%3: it is read by QK at half-steps 2u-1 and 2u and by PV
-    // at 2u+1 and 2u+2, and its halves are written at 2u-3 (group 1) and 2u-2 (group 0),
-    // when the tile that used the buffer before (u-3) is no longer read.  A group's raw
-    // register set holds its half of two tiles in flight (even tiles in one set, odd in
-    // the other), so a load has two tiles' time to arrive.  Group g dequantizes / fetches
-    // as thread tid ^ 256, which maps group 0 to entries 16..31 and group 1 to 0..15.
-    Piece raw[RP::PPT];
-    int g_pref = -1;
-    const int ptid = tid ^ 256;
-    auto ktile = [&](int u) __attribute__((always_inline)) -> uint8_t* { return kt0 + (u % 3) * M::KT; };
-
-    // softmax of tile u for this wave's heads: S^T partials -> running max / sum -> P^T
-    // The softmax runs at a raised wave priority: on its SIMD the other group's wave is in
-    // its MFMA half-step, whose issue slots the softmax's dependent LDS reads and exps then
-    // win (the MFMA chain waits on its own operand reads most of the time).  Measured: 72.4
-    // -> 71.6 us per config-2 step; the priority over the whole traffic half-step (stores
-    // and gathers too), or on the MFMA half-step instead, was no better or slower.
-    auto softmax = [&](int u) __attribute__((always_inline)) {
-      __builtin_amdgcn_s_setprio(1);
-      const uint32_t vmask = tab_mask[u & rp.slot_mask];
-      // entries 8ds..8ds+7 of tile u for this lane's head
-      float4 a = sx[((hg * DS) * 4 + ds) * 64 + lane];
-#pragma unroll
-      for (int part = 1; part < DS; ++part) {
-        const float4 c = sx[((hg * DS + part) * 4 + ds) * 64 + lane];
-        a.x = a.x + c.x;
-        a.y = a.y + c.y;
-        a.z = a.z + c.z;
-        a.w = a.w + c.w;
-      }
-      float v4[4] = {a.x * p.scale_log2, a.y * p.scale_log2, a.z * p.scale_log2, a.w * p.scale_log2};
-      if (vmask != 0xffffffffu) {
-        const uint32_t bits = vmask >> (8 * ds + 4 * half);  // entries 8ds + 4half + i
-#pragma unroll
-        for (int i = 0; i < 4; ++i)
-          if (!((bits >> i) & 1u)) v4[i] = -__builtin_huge_valf();
-      }
-      const float lane_max = fmaxf(fmaxf(v4[0], v4[1]), fmaxf(v4[2], v4[3]));
-      float bound;
-      if constexpr (kExact) {
-        // the head's true tile max: its 8 lanes' maxima through LDS (the other group
-        // passes the matching barrier at the start of its MFMA half-step)
-        pe[pm_slot] = lane_max;
-        lds_barrier();
-        const float4 t0 = reinterpret_cast<const float4*>(pe)[hl];
-        const float4 t1 = reinterpret_cast<const float4*>(pe)[64 + hl];
-        bound = fmaxf(fmaxf(fmaxf(t0.x, t0.y), fmaxf(t0.z, t0.w)), fmaxf(fmaxf(t1.x, t1.y), fmaxf(t1.z, t1.w)));
-      } else {
-        m_seen = fmaxf(m_seen, lane_max);
-        const float4 t0 = reinterpret_cast<const float4*>(pm)[hl];
-        const float4 t1 = reinterpret_cast<const float4*>(pm)[64 + hl];
-        bound = (((fmaxf(t0.x, t0.y) + fmaxf(t0.z, t0.w)) + fmaxf(t1.x, t1.y)) + fmaxf(t1.z, t1.w)) * p.scale_log2;
-      }
-      const bool raise = bound > m_run + kLazy;
-      if (__any(raise)) {  // identical in every wave of the head group
-        const float m_new = raise ? bound : m_run;
-        const float alpha = (m_run == -__builtin_huge_valf()) ? 0.0f : __builtin_amdgcn_exp2f(m_run - m_new);
-        l_run = l_run * alpha;
-#pragma unroll
-        for (int i = 0; i < NDBM; ++i) acc_o[i] = acc_o[i] * alpha;
-        m_run = m_new;
-      }
-      // the exact pass may see a head with no finite entry yet (m_run = -inf): then every
-      // entry is -inf and the reference point 0 gives exp2(-inf) = 0 instead of NaN
-      const float m_use = (kExact && m_run == -__builtin_huge_valf()) ? 0.0f : m_run;
-      const float p0 = __builtin_amdgcn_exp2f(v4[0] - m_use);
-      const float p1 = __builtin_amdgcn_exp2f(v4[1] - m_use);
-      const float p2 = __builtin_amdgcn_exp2f(v4[2] - m_use);
-      const float p3 = __builtin_amdgcn_exp2f(v4[3] - m_use);
-      l_run = l_run + ((p0 + p1) + (p2 + p3));
-      // PV K-step ks = ds/2 takes registers 8ks..8ks+7 = D-parts 2ks (slots 0-3), 2ks+1 (4-7)
-      uint2* dst = reinterpret_cast<uint2*>(pb + (hg * 2 + (ds >> 1)) * 64 + lane) + (ds & 1);
-      *dst = uint2{pack_bf16x2(p0, p1), pack_bf16x2(p2, p3)};
-      __builtin_amdgcn_s_setprio(0);
-    };
-    // O^T += V^T.P^T of tile `u` (if pv) and the S^T partial of tile u+1 (if qk), in one
-    // block so the two MFMA streams interleave.  Near the end QK runs on a stale buffer;
-    // its partial is published but never read.
-    auto mfma_step = [&](int u, bool pv, bool qk_next) __attribute__((always_inline)) {
-      if constexpr (kExact) lds_barrier();  // pairs with the exact softmax's barrier
-      // Software pipeline for a lone MFMA wave: every operand is read from LDS a step
-      // ahead of the MFMA that consumes it (V^T one 32-channel block ahead, K two K-steps
-      // ahead), and scheduling fences keep the compiler from collapsing the pipeline.
-      const uint8_t* kt_q = ktile(u + 1) + (lane & 31) * KT_PITCH + 2 * (qc0 + half * 8);
-      constexpr int NB_MIN = NB / DS;  // O^T blocks every wave owns (the last one may own one more)
-      uint4 kv[QST];
-      v16f s_acc = v16f{};
-      // one QK K-step; K fragments are read two steps ahead (compile-time indices only)
-      auto qk_step = [&](int st) __attribute__((always_inline)) {
-        if (st + 2 < QST) kv[st + 2] = *reinterpret_cast<const uint4*>(kt_q + 32 * (st + 2));
-        s_acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
-            __builtin_bit_cast(v8bf, v4i{(int)kv[st].x, (int)kv[st].y, (int)kv[st].z, (int)kv[st].w}), qf[st], s_acc,
-            0, 0, 0);
-      };
-      if (qk_next) {
-        kv[0] = *reinterpret_cast<const uint4*>(kt_q);
-        if (QST > 1) kv[1] = *reinterpret_cast<const uint4*>(kt_q + 32);
-      }
-      if (pv) {
-        const uint4 w0 = pb[(hg * 2 + 0) * 64 + lane];
-        const uint4 w1 = pb[(hg * 2 + 1) * 64 + lane];
-        const v8bf pf0 = __builtin_bit_cast(v8bf, v4i{(int)w0.x, (int)w0.y, (int)w0.z, (int)w0.w});
-        const v8bf pf1 = __builtin_bit_cast(v8bf, v4i{(int)w1.x, (int)w1.y, (int)w1.z, (int)w1.w});
-        const uint8_t* tr0 = ktile(u) + pv_off;
-        // V^T operands double-buffered by block parity, so block db+1's reads are in flight
-        // while block db's MFMAs run
-        v4s rv[2][4];
-        auto read_v = [&](int db) __attribute__((always_inline)) {
-          const uint8_t* tp = tr0 + 64 * db;
-          v4s (&r)[4] = rv[db & 1];
-          r[0] = __builtin_amdgcn_ds_read_tr16_b64_v4i16(lds_v4s(tp));
-          r[1] = __builtin_amdgcn_ds_read_tr16_b64_v4i16(lds_v4s(tp + 8 * KT_PITCH));
-          r[2] = __builtin_amdgcn_ds_read_tr16_b64_v4i16(lds_v4s(tp + 16 * KT_PITCH));
-          r[3] = __builtin_amdgcn_ds_read_tr16_b64_v4i16(lds_v4s(tp + 24 * KT_PITCH));
-        };
-        // PV of block db; with_qk interleaves K-steps 2db and 2db+1 of QK (compile time)
-        auto pv_mfma = [&](int db, bool more, bool with_qk) __attribute__((always_inline)) {
-          if (more) read_v(db + 1);
-          const v4s (&r)[4] = rv[db & 1];
-          const v8bf a0 = __builtin_bit_cast(v8bf, v8s{r[0][0], r[0][1], r[0][2], r[0][3], r[1][0], r[1][1], r[1][2], r[1][3]});
-          const v8bf a1 = __builtin_bit_cast(v8bf, v8s{r[2][0], r[2][1], r[2][2], r[2][3], r[3][0], r[3][1], r[3][2], r[3][3]});
-          acc_o[db] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a0, pf0, acc_o[db], 0, 0, 0);
-          if (with_qk && qk_next && 2 * db < QST) qk_step(2 * db);
-          acc_o[db] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a1, pf1, acc_o[db], 0, 0, 0);
-          if (with_qk && qk_next && 2 * db + 1 < QST) qk_step(2 * db + 1);
-          __builtin_amdgcn_sched_barrier(0);
-        };
-        read_v(0);
-#pragma unroll
-        for (int db = 0; db < NB_MIN; ++db) pv_mfma(db, db + 1 < NB_MIN || nb_mine > NB_MIN, true);
-        static_assert(2 * NB_MIN <= QST, "every interleaved K-step index must exist");
-#pragma unroll
-        for (int st = 2 * NB_MIN; st < QST; ++st)
-          if (qk_next) qk_step(st);
-        if (nb_mine > NB_MIN) {  // the wave's extra block: the K-steps above are all issued
-#pragma unroll
-          for (int db = NB_MIN; db < NDBM; ++db) pv_mfma(db, false, false);
-        }
-      } else if (qk_next) {
-#pragma unroll
-        for (int st = 0; st < QST; ++st) qk_step(st);
-      }
-      if (qk_next) publish(s_acc);
-    };
-    // group 0: even(u) softmax + traffic, odd(u) PV(u) + QK(u+1)
-    auto group0_pair = [&](int u, Piece (&r0)[RP::PPT]) {
-      lds_barrier();
-      softmax(u);
-      rp.store(ktile(u + 1), KT_PITCH, ptid, r0);
-      // the index of tile u+5 is read before the fetch is issued: the wait on that read
-      // (the compiler's counters are in order) then covers no fetch load
-      const int g_next = !all_tables && tid < kTile ? rp.slot(rp.v_begin + (u + 5) * kTile + tid) : -1;
-      rp.fetch(u + 2, ptid, r0);
-      if (!all_tables) rp.build_table(p, u + 4, g_pref, tid);
-      g_pref = g_next;
-      lds_barrier();
-      mfma_step(u, true, true);
-    };
-    // group 1: even(u) PV(u-1) + QK(u), odd(u) softmax + traffic
-    auto group1_pair = [&](int u, Piece (&r1)[RP::PPT]) {
-      lds_barrier();
-      mfma_step(u - 1, true, true);
-      lds_barrier();
-      softmax(u);
-      rp.store(ktile(u + 2), KT_PITCH, ptid, r1);
-      rp.fetch(u + 3, ptid, r1);
-    };
-    if (rp.ntiles > 0) {
-      if (!all_tables) {
-        rp.build_first_tables(p, tid);
-        if (tid < kTile) g_pref = rp.slot(rp.v_begin + 4 * kTile + tid);
-      }
-      __syncthreads();
-      rp.fetch(0, ptid, raw);
-      if constexpr (!kExact && RST > 0) {
-        // q's rope steps are rotated while tile 0's gathers are in flight (q and the tables
-        // were requested before them, so the wait covers no gather)
-        if (q_rope) {
-#pragma unroll
-          for (int r = 0; r < RST; ++r) {
-            v4i v = __builtin_bit_cast(v4i, qf[QST - RST + r]);
-            const uint32_t cw_[2] = {qrc[r].x, qrc[r].y}, sw_[2] = {qrs[r].x, qrs[r].y};
-#pragma unroll
-            for (int k = 0; k < 4; ++k) {
-              const uint32_t cp = cw_[k >> 1], sp = sw_[k >> 1];
-              v[k] = static_cast<int>(rope_pair_bf16(static_cast<uint32_t>(v[k]),
-                                                     bf16_to_f32(static_cast<uint16_t>((k & 1) ? cp >> 16 : cp & 0xffffu)),
-                                                     bf16_to_f32(static_cast<uint16_t>((k & 1) ? sp >> 16 : sp & 0xffffu))));
-            }
-            qf[QST - RST + r] = __builtin_bit_cast(v8bf, v);
-          }
-        }
-      }
-      rp.store(ktile(0), KT_PITCH, ptid, raw);
-      rp.fetch(1, ptid, raw);
-      if (hg == 1) {  // group 1 also writes its half of tile 1 and holds tile 2
-        rp.store(ktile(1), KT_PITCH, ptid, raw);
-        rp.fetch(2, ptid, raw);
-      }
-      lds_barrier();  // tile 0 and half of tile 1 complete
-      if (hg == 0) publish(qk(ktile(0)));
-    }
-    // group 0 dequantizes tile u+1 from set (u+1)&1, group 1 tile u+2 from set u&1
-    // the loops execute the same barriers in the same order (two per tile, three in the
-    // exact pass)
-    if (hg == 0) {
-#pragma unroll 1
-      for (int u = 0; u < rp.ntiles; ++u) group0_pair(u, raw);
-    } else if (rp.ntiles > 0) {
-      // u = 0: no PV yet, QK(0) only
-      lds_barrier();
-      mfma_step(-1, false, true);
-      lds_barrier();
-      softmax(0);
-      rp.store(ktile(2), KT_PITCH, ptid, raw);
-      rp.fetch(3, ptid, raw);
-#pragma unroll 1
-      for (int u = 1; u < rp.ntiles; ++u) group1_pair(u, raw);
-    }
-    if (rp.ntiles > 0) {
-      lds_barrier();  // even(nt): the last P^T of group 1 complete
-      if (hg == 1) mfma_step(rp.ntiles - 1, true, false);
-      else if constexpr (kExact) lds_barrier();
-    }
-
-    // row sum: each lane holds the share of its entries (all scaled to the same running
-    // max); the 8 shares of a head are reduced in a fixed order
-    __syncthreads();  // every wave is done reading pm and pe
-    pm[pm_slot] = l_run;
-    if (!kExact) pe[pm_slot] = m_seen;
-    __syncthreads();
-    {
-      const float4 t0 = reinterpret_cast<const float4*>(pm)[hl];
-      const float4 t1 = reinterpret_cast<const float4*>(pm)[64 + hl];
-      l_run = (((t0.x + t0.y) + (t0.z + t0.w)) + ((t1.x + t1.y) + (t1.z + t1.w)));
-    }
-    if constexpr (!kExact) {
-      const float4 t0 = reinterpret_cast<const float4*>(pe)[hl];
-      const float4 t1 = reinterpret_cast<const float4*>(pe)[64 + hl];
-      const float m_true =
-          fmaxf(fmaxf(fmaxf(t0.x, t0.y), fmaxf(t0.z, t0.w)), fmaxf(fmaxf(t1.x, t1.y), fmaxf(t1.z, t1.w)));
-      // a head with no unmasked entry (m_true = -inf) contributes nothing and is exact
-      if (head_ok && m_true > -__builtin_huge_valf() && m_run - m_true > kBoundSlack) redo = 1;
-      __syncthreads();
-      if (redo) return false;  // uniform: every wave reads the flag after the same barrier
-    }
-    if (head_ok)
-      write_result<D, NOPE, NDBM>(p, rp.row, rp.b, rp.split, head, half, ds == 0 && half == 0, b_lo, nb_mine, m_run, l_run,
-                            acc_o);
-    return true;
-  };
-
-  if (!pass(std::false_type{})) pass(std::true_type{});
-  if constexpr (ALLTAB) {
-    if (mrec != nullptr) merge_in_launch<D, NOPE, NT>(p, rp.row, rp.hgrp * HG * 32, rp.split, mrec, tid);
-  }
-}
+#include "attention_latent.h"
 
 // positions[i] += 1 for the rows of a call whose last launch does not merge splits.
 __global__ void __launch_bounds__(256) advance_kernel(int64_t* __restrict__ positions, int64_t rows) {
@@ -1607,16 +1005,6 @@ int launch_kernel(K kern, size_t dyn_lds, int threads, int heads_per_wg, const A
   return MZK_OK;
 }
 
-// Whether the longest split any workgroup of a D-split launch can plan (RowPlan::plan with
-// every source full) keeps all its entry tables (RowPlan::table_tiles): the decode kernel
-// instances (ALLTAB), which the in-launch merge and the in-launch selection need.
-bool dsplit_all_tables(int window, const void* dense, int dense_cap, const void* main_kv, int topk, int nsplit) {
-  const int64_t total_max = static_cast<int64_t>(window) + (dense ? dense_cap : 0) + (main_kv ? topk : 0);
-  const int64_t chunk_max = ((total_max + nsplit - 1) / nsplit + kTile - 1) / kTile * kTile;
-  const int64_t tables_max = chunk_max / kTile + 3 > 4 ? chunk_max / kTile + 3 : 4;
-  return tables_max * kTile <= kAllTabCap;
-}
-
 // `merged` is set when the launch merges its splits itself (p.merge_rec given and the
 // launch takes the kernel instance that carries the merge).
 template <int FMT, int D, int NOPE>
@@ -1628,12 +1016,9 @@ int dispatch_heads(const AttnParams& p_in, int64_t rows, hipStream_t s, bool* me
     return MZK_EUNSUPPORTED;
   }
   if constexpr (D > 256) {
-    // 64 heads per workgroup, each 32-head group split by D over 4 waves
-    using M = SplitSmem<FMT, D, NOPE>;
-    static_assert(M::LDS + 8 * kAllTabCap + 4 * (kAllTabCap / kTile) + 128 <= 160 * 1024, "LDS budget");
-    auto kern_all = sparse_mqa_dsplit_kernel<FMT, D, NOPE, true>;
-    auto kern_ring = sparse_mqa_dsplit_kernel<FMT, D, NOPE, false>;
-    auto kern_sel = sparse_mqa_dsplit_kernel<FMT, D, NOPE, true, true>;
+    static_assert(D == LatentSmem::D && LatentSmem::LDS <= 160 * 1024, "the latent kernel's shape and LDS budget");
+    auto kern = sparse_mqa_latent_kernel<FMT, NOPE, false>;
+    auto kern_sel = sparse_mqa_latent_kernel<FMT, NOPE, true>;
     // the dynamic-LDS limit is a per-device function attribute: set once per device
     static std::atomic<bool> attr_set[kMaxDevices] = {};  // setting it twice is harmless
     int dev = 0;
@@ -1642,27 +1027,16 @@ int dispatch_heads(const AttnParams& p_in, int64_t rows, hipStream_t s, bool* me
       return MZK_ELAUNCH;
     }
     if (!attr_set[dev].load(std::memory_order_acquire)) {
-      for (const void* k : {reinterpret_cast<const void*>(kern_all), reinterpret_cast<const void*>(kern_ring),
-                            reinterpret_cast<const void*>(kern_sel)}) {
-        if (hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, M::LDS) != hipSuccess) {
-          set_last_error("sparse_mqa: cannot raise the kernel's LDS limit to %d bytes", M::LDS);
+      for (const void* k : {reinterpret_cast<const void*>(kern), reinterpret_cast<const void*>(kern_sel)}) {
+        if (hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, LatentSmem::LDS) != hipSuccess) {
+          set_last_error("sparse_mqa: cannot raise the kernel's LDS limit to %d bytes", LatentSmem::LDS);
           return MZK_ELAUNCH;
         }
       }
       attr_set[dev].store(true, std::memory_order_release);
     }
-    const bool all_tables = dsplit_all_tables(p.window, p.dense, p.dense_cap, p.main, p.topk, p.nsplit);
-    if (!all_tables) p.merge_rec = nullptr;  // only the decode instance carries the in-launch merge
-    if (p.sel_scores != nullptr) {  // the host checked the selecting instance's limits
-      if (!all_tables) {
-        set_last_error("sparse_mqa_select: the splits exceed the decode kernel's entry tables");
-        return MZK_EUNSUPPORTED;
-      }
-      *merged = p.merge_rec != nullptr;
-      return launch_kernel(kern_sel, M::LDS, 512, 64, p, rows, s);
-    }
     *merged = p.merge_rec != nullptr;
-    return launch_kernel(all_tables ? kern_all : kern_ring, M::LDS, 512, 64, p, rows, s);
+    return launch_kernel(p.sel_scores != nullptr ? kern_sel : kern, LatentSmem::LDS, 256, 64, p, rows, s);
   } else {
     if (p.H <= 32) return launch_kernel(sparse_mqa_kernel<FMT, D, NOPE, 1>, 0, 64, 32, p, rows, s);
     return launch_kernel(sparse_mqa_kernel<FMT, D, NOPE, 2>, 0, 128, 64, p, rows, s);
@@ -1849,7 +1223,7 @@ int sparse_mqa_impl(const void* q, int64_t B, int64_t S, int H, int D, int fmt, 
   p.sel_out = sel_out;
   p.sel_out_stride = sel_out_stride;
   if (sel_scores) p.idx = nullptr;
-  // The split merge inside the attention launch: a full call of the D-split kernel with
+  // The split merge inside the attention launch: a full call of the latent kernel with
   // nsplit dividing 64, rows or rows * (64-head groups) a multiple of 8 (the mappings that put
   // a group's splits on one XCD), a workspace that holds the merge records, and a grid of at
   // most one workgroup per CU (every workgroup of a group must run at once; one fills a CU's
@@ -1972,13 +1346,11 @@ extern "C" int mzk_sparse_mqa_select(const void* q, int64_t B, int H, int D, int
                 "sparse_mqa_select: out and lse, or neither (split partials only: nsplit > 1, no advance)");
   MZK_CHECK_ARG(score_stride >= G && idx_out_stride >= topk, "sparse_mqa_select: strides smaller than the row");
   if (B == 0) return MZK_OK;
-  // the selecting kernel instance: the FP8 latent decode kernel, 16 scores per thread of its
-  // 512, whole float4 / int4 groups
+  // the selecting kernel instance: the FP8 latent kernel, 32 scores per thread of its 256,
+  // whole float4 / int4 groups
   const bool in_launch = fmt == 1 && D == 576 && nope == 512 && G >= 4 && G <= 8192 && G % 4 == 0 &&
                          score_stride % 4 == 0 && aligned16(scores) && topk >= 4 && topk <= 2048 && topk % 4 == 0 &&
-                         idx_out_stride % 4 == 0 && aligned16(idx_out) && nsplit >= 1 && nsplit <= 65535 &&
-                         window >= 0 && dense_cap >= 0 &&
-                         dsplit_all_tables(window, dense, dense_cap, main_kv, topk, nsplit);
+                         idx_out_stride % 4 == 0 && aligned16(idx_out);
   int64_t* adv = advance ? positions : nullptr;
   if (!in_launch) {  // the top-k launch, then the attention over its list
     int rc = mzk_topk_rows(scores, B, G, score_stride, topk, idx_out, idx_out_stride, stream);

@@ -305,6 +305,11 @@ __device__ __forceinline__ float exp_pinned(float x) {
   return out;
 }
 
+// Workgroup barrier that waits only for this wave's LDS operations (not for vector
+// memory: the next tile's loads stay in flight across it).  The "memory" clobber keeps
+// the compiler from moving memory accesses across.
+__device__ __forceinline__ void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" : : : "memory"); }
+
 // ------------------------------------------------------------------------------------
 // wave helpers (wave64)
 // ------------------------------------------------------------------------------------

@@ -14,7 +14,8 @@
 // are what a level costs.  The selection (owlet1/indexer.py:158-165 with a deterministic tie
 // rule): key > T, and the first need_eq keys equal to T in index order; the output slot of a
 // taken key is (#key > T before it) + min(#key == T before it, need_eq), from one scan of the
-// packed pair (n_gt << 16 | n_eq).
+// packed pair (n_gt << 16 | n_eq).  The barriers wait for LDS operations only: whatever the
+// caller has requested from memory stays in flight across them.
 #pragma once
 
 #include "common.h"
@@ -60,7 +61,7 @@ __device__ __forceinline__ int block_incl_scan(int v, int* wsum, int& total) {
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int incl = wave_incl_scan_dpp(v);
   if (lane == 63) wsum[wave] = incl;
-  __syncthreads();
+  lds_barrier();
   int before = 0, tot = 0;
 #pragma unroll
   for (int w = 0; w < NW; ++w) {
@@ -103,7 +104,7 @@ __device__ __forceinline__ BinHit find_bin(const int (&c)[NB / NT], int rem, int
     }
     above += c[j];
   }
-  __syncthreads();
+  lds_barrier();
   return BinHit{sh[0], sh[1], sh[2], total};
 }
 
@@ -149,7 +150,7 @@ __device__ __forceinline__ void row_sel_threshold(const uint32_t (&key)[KPT], bo
 #pragma unroll
     for (int j = 0; j < KPT; ++j)
       if (key[j] > kNegInfKey) atomicAdd(hl + (key[j] >> kLowBits) * kSub1, 1);
-    __syncthreads();
+    lds_barrier();
     int c1[BPT];
 #pragma unroll
     for (int j = 0; j < BPT; ++j) {
@@ -174,7 +175,7 @@ __device__ __forceinline__ void row_sel_threshold(const uint32_t (&key)[KPT], bo
 #pragma unroll
       for (int j = 0; j < KPT; ++j)
         if ((key[j] >> kLowBits) == b1) atomicAdd(&s.hist2[(key[j] >> 10) & (kBins - 1)], 1);
-      __syncthreads();
+      lds_barrier();
       int c2[BPT];
 #pragma unroll
       for (int j = 0; j < BPT; ++j) c2[j] = s.hist2[kBins - 1 - (BPT * tid + j)];
@@ -186,7 +187,7 @@ __device__ __forceinline__ void row_sel_threshold(const uint32_t (&key)[KPT], bo
 #pragma unroll
         for (int j = 0; j < KPT; ++j)
           if ((key[j] >> 10) == (p2 >> 10)) atomicAdd(&s.hist3[key[j] & 1023u], 1);
-        __syncthreads();
+        lds_barrier();
         constexpr int B3 = kBins / 2;
         int c3[B3 / NT];
 #pragma unroll
