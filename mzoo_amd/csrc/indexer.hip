@@ -862,198 +862,303 @@ __global__ void __launch_bounds__(kWaves * 64) indexer_scores_kernel(const IdxPa
 
 
 // ------------------------------------------------------------------------------------
-// Prefill form (FP8, Di = 128): many query rows against the same keys.  The decode tiling
-// re-streams every key for every query row; here one workgroup takes kPfQb query rows and
-// walks the key blocks of 512: per block a wave holds 128 keys (4 N-blocks of 32, two
-// 64-channel steps) as the MFMA B operand and runs the rows through them (A = a row's 64
-// heads as two 32-row M-blocks).  The rows' codes are staged in LDS once, at the start (one
-// memory round trip; 144-byte row pitch against bank conflicts), with the per-head weights
-// w * q_scale next to them; each lane reads the 16 accumulator rows it holds.  Within a
-// row the next key tile's MFMAs are issued while the current tile's ReLU-weighted head sum
-// runs (the two take about as long).  Keys a row cannot see (at or beyond (pos + 1) //
-// ratio) are written as -inf without MFMA work, blocks beyond every row's visibility
-// without loading them, and the workgroups with the most visible keys are dispatched first
-// (the grid runs the query blocks from the last to the first).  The head sum runs in the
-// row kernel's order, so the scores are the row kernel's bit for bit.
+// Prefill form (FP8 and MXFP4, Di = 128): many query rows against the same keys.  The decode
+// tiling re-streams every key for every query row; here a wave keeps kUnits = 4 query blocks
+// of 32 heads (2 rows of 64 heads, or 4 rows of 32) in registers, fragments and head
+// weights, and the keys stream past: the workgroup's four waves (8 or 16 rows) share each
+// chunk of 128 keys through LDS.
+//
+// What bounds it is the vector unit: the ReLU-weighted head sum takes two operations per
+// (head, key), 128 cycles per query block and 32-key tile on a SIMD, where the block's two
+// FP8 MFMAs take 128 cycles (MXFP4 64) of the matrix unit.  So the loop is one chain of
+// (tile, block) units that never drains, across tiles and chunks: the next unit's MFMAs are
+// issued inside the current unit's head sum (two accumulators of 16 registers in turn), the
+// next tile's key fragments are read from LDS a tile ahead and the chunk after next is
+// requested from memory a chunk ahead.  8192 causal rows of 64 heads, 2048 FP8 keys: 106 ->
+// 73 us, about 23 of them the query's and the scores' memory traffic and the rest within
+// 1.2 times of the head sums alone.  (The earlier form kept 4 key tiles in registers and
+// re-read every row's fragments and weights from LDS between drained pipelines: matrix unit
+// busy 32 % and vector unit 44 % of the time.)  1021 rows of 32 heads on 4004 MXFP4 keys,
+// which the row form served before: 35 -> 18.8 us.  Taken back: pinning one MFMA to 16 vector
+// operations (2 % slower), storing the -inf of the unseen keys from inside the loop (5 %
+// slower), 3 or 4 workgroups per compute unit's worth of key splits (up to 20 % slower where
+// the rows are few).
+//
+// LDS: three chunk buffers, one barrier per chunk.  Chunk c + 1 is written between the
+// barriers of chunks c - 1 and c, over chunk c - 2, whose reads every wave had finished
+// before the barrier of c - 1.  A key's 16-byte pieces are stored exclusive-or a key number
+// so that each phase of a fragment read meets all 64 banks.
+//
+// The head sum runs in the row kernel's order, so the scores are the row kernel's bit for
+// bit.  Keys a row cannot see (at or beyond (pos + 1) // ratio) are written as -inf; chunks
+// that no row of the workgroup sees get no MFMA work.  The row blocks are dispatched from the
+// last, whose rows see the most keys.
 // ------------------------------------------------------------------------------------
-constexpr int kPfQb = 8;               // query rows per workgroup
 constexpr int kPfPrefillMinRows = 64;  // rows per batch from which the prefill form is used
-constexpr int kPfPitch = 144;          // LDS bytes per staged head row
-constexpr int kPfLds = kPfQb * 64 * kPfPitch + kPfQb * 64 * 4 + kPfQb * 8;
+constexpr int kPfChunk = 128;          // keys per staged chunk
+constexpr int kPfUnits = 4;            // query blocks of 32 heads per wave
 
-__global__ void __launch_bounds__(kWaves * 64, 2) indexer_prefill_fp8_kernel(const IdxParams p, int64_t nqb) {
-  constexpr int DI = 128, NST = 2;
-  extern __shared__ __align__(16) uint8_t pf_smem[];
-  uint8_t* q_lds = pf_smem;                                                   // [qb][64][kPfPitch]
-  float* coef_lds = reinterpret_cast<float*>(pf_smem + kPfQb * 64 * kPfPitch);  // [qb][64]
-  int64_t* vis_lds = reinterpret_cast<int64_t*>(coef_lds + kPfQb * 64);        // [qb]
+template <int FMT>
+struct PfChunk {
+  static constexpr int RB = row_bytes<FMT>(kDi);
+  static constexpr int kPieces = kPfChunk * RB / 16 / (kWaves * 64);  // 16-byte pieces per thread
+  static constexpr int kKx = kPfChunk * RB;                           // the keys' scale words
+  static constexpr int kBytes = kKx + 4 * kPfChunk;
+};
+
+template <int FMT, int MB>
+__global__ void __launch_bounds__(kWaves * 64, 2)
+    indexer_prefill_kernel(const IdxParams p, int nrb, int nsplit, int split_chunks) {
+  constexpr int DI = kDi, NST = DI / Step<FMT>::K;
+  constexpr int RW = kPfUnits / MB;  // query rows per wave
+  constexpr int QB = kWaves * RW;    // and per workgroup
+  constexpr int NP = RW / 2;         // row pairs per wave
+  using C = PfChunk<FMT>;
+  constexpr int RB = C::RB;
+  static_assert(FMT == kFp8 || FMT == kMxfp4, "quantized operands");
+  __shared__ __align__(16) uint8_t kbuf[3 * C::kBytes];
+  __shared__ __align__(16) float coef_lds[kWaves][kPfUnits * 32];
   const int tid = threadIdx.x;
   const int lane = tid & 63;
-  const int wave = tid >> 6;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int hi = lane >> 5;
-  const int64_t nkb = (p.G + kKeysPerWg - 1) / kKeysPerWg;
-  const int64_t qb_all = static_cast<int64_t>(gridDim.x) - 1 - blockIdx.x;  // last query block first
-  const int64_t b = qb_all / nqb;
-  const int64_t s0 = (qb_all % nqb) * kPfQb;
+  const int col = lane & 31;
   const int Hi = p.Hi;
-  const int64_t G = p.G, S = p.S;
-  const float inv_sqrt_di = 1.0f / sqrt_rn(static_cast<float>(DI));
-  const int nq = static_cast<int>(S - s0 < kPfQb ? S - s0 : kPfQb);
-  const uint8_t* kb_base = p.k + b * p.kbs * DI;
-  const float* ks_base = p.k_scale + b * p.kbs;
-  // the rows' codes: 16-byte piece i = (row, head, piece) of the block, every load issued
-  // before any is stored (rows beyond the block and heads beyond Hi read row 0 / head 0 and
-  // store zeros)
-  constexpr int kPieces = kPfQb * 64 * (DI / 16);
-  constexpr int kPerThread = kPieces / (kWaves * 64);
-  uint4 pc[kPerThread];
-#pragma unroll
-  for (int k = 0; k < kPerThread; ++k) {
-    const int i = tid + k * kWaves * 64;
-    const int qi = i / (64 * (DI / 16)), h = (i / (DI / 16)) % 64, c = i % (DI / 16);
-    const bool ok = qi < nq && h < Hi;
-    const int64_t r = b * S + s0 + (ok ? qi : 0);
-    pc[k] = *reinterpret_cast<const uint4*>(p.q + (r * Hi + (ok ? h : 0)) * DI + 16 * c);
-  }
-  for (int i = tid; i < kPfQb * 64; i += kWaves * 64) {
-    const int qi = i >> 6, h = i & 63;
-    float c = 0.0f;
-    if (qi < nq && h < Hi) {
-      const int64_t r = b * S + s0 + qi;
-      c = p.w[r * Hi + h] * p.q_scale[r * Hi + h];
-    }
-    coef_lds[i] = c;
-  }
-  if (tid < kPfQb) {
-    int64_t v = 0;
-    if (tid < nq) {
-      const int64_t r = b * S + s0 + tid;
-      const int64_t pos = p.positions ? p.positions[r] : s0 + tid;
-      v = (pos + 1) / p.ratio;
-      v = v > G ? G : (v < 0 ? 0 : v);
-    }
-    vis_lds[tid] = v;
-  }
-#pragma unroll
-  for (int k = 0; k < kPerThread; ++k) {
-    const int i = tid + k * kWaves * 64;
-    const int qi = i / (64 * (DI / 16)), h = (i / (DI / 16)) % 64, c = i % (DI / 16);
-    const bool ok = qi < nq && h < Hi;
-    *reinterpret_cast<uint4*>(q_lds + (qi * 64 + h) * kPfPitch + 16 * c) = ok ? pc[k] : uint4{0u, 0u, 0u, 0u};
-  }
-  __syncthreads();
-  int64_t vis_max = 0;
-  for (int qi = 0; qi < nq; ++qi) vis_max = vis_lds[qi] > vis_max ? vis_lds[qi] : vis_max;
+  const int G = static_cast<int>(p.G);
+  const int blk = static_cast<int>(gridDim.x - 1 - blockIdx.x);  // the last row block first
+  const int rb_all = blk / nsplit;
+  const int split = blk - rb_all * nsplit;
+  const int64_t b = rb_all / nrb;
+  const int64_t s0 = static_cast<int64_t>(rb_all - b * nrb) * QB;
+  const int nq = static_cast<int>(p.S - s0 < QB ? p.S - s0 : QB);
+  const int64_t row0 = b * p.S + s0;  // the workgroup's first query row
+  const uint8_t* kb = p.k + b * p.kbs * RB;
+  // the keys' scale words: the fp32 scale, or the key's four e8m0 bytes
+  const uint32_t* kx = FMT == kFp8 ? reinterpret_cast<const uint32_t*>(p.k_scale + b * p.kbs)
+                                   : reinterpret_cast<const uint32_t*>(p.k_e8m0 + b * p.kbs * (DI / 32));
 
-  // the key blocks in turn: every block with a visible key is scored, and the blocks
-  // beyond every row's visibility are written as -inf
-  for (int64_t kb = 0; kb < nkb; ++kb) {
-    const int64_t key0 = kb * kKeysPerWg + wave * (kNkb * 32);
-    if (kb * kKeysPerWg >= vis_max) {
-      if (lane < 32) {
-        for (int qi = 0; qi < nq; ++qi) {
-          float* out = p.scores + (b * S + s0 + qi) * p.sstride;
+  // every load before anything waits for one: the positions, the first chunk, the query
+  int64_t pos = s0 + lane;
+  if (p.positions && lane < nq) pos = p.positions[row0 + lane];
+  const int c0 = split * split_chunks;
+  const int kend = (c0 + split_chunks) * kPfChunk < G ? (c0 + split_chunks) * kPfChunk : G;  // the split's key range
+  // one chunk: kPieces coalesced 16-byte pieces and a key's scale word per thread; keys at or beyond G read key G - 1, their columns are never written
+  constexpr int kPerKey = RB / 16;                     // pieces of a key
+  constexpr int kStride = kWaves * 64 / kPerKey;       // keys between a thread's pieces
+  const int lkey = tid / kPerKey, lpc = tid % kPerKey;
+  const int lsw = (tid >> 4) & (kPerKey - 1);          // pitch 128: (key >> 1) & 7; 64: (key >> 2) & 3
+  const int lds_at = lkey * RB + ((lpc ^ lsw) << 4);
+  struct Stage {
+    v4i v[C::kPieces];
+    uint32_t x;
+  };
+  auto fetch = [&](int c) __attribute__((always_inline)) {
+    Stage sg;
 #pragma unroll
-          for (int t = 0; t < kNkb; ++t) {
-            const int64_t g = key0 + t * 32 + lane;
-            if (g < G) out[g] = -__builtin_huge_valf();
-          }
+    for (int i = 0; i < C::kPieces; ++i) {
+      int key = c * kPfChunk + i * kStride + lkey;
+      key = key < G ? key : G - 1;
+      sg.v[i] = *reinterpret_cast<const v4i*>(kb + static_cast<int64_t>(key) * RB + 16 * lpc);
+    }
+    int key = c * kPfChunk + (tid & (kPfChunk - 1));
+    key = key < G ? key : G - 1;
+    sg.x = kx[key];
+    return sg;
+  };
+  auto put = [&](int base, const Stage& sg) __attribute__((always_inline)) {
+#pragma unroll
+    for (int i = 0; i < C::kPieces; ++i)
+      *reinterpret_cast<v4i*>(kbuf + base + lds_at + i * kStride * RB) = sg.v[i];
+    *reinterpret_cast<uint32_t*>(kbuf + base + C::kKx + 4 * (tid & (kPfChunk - 1))) = sg.x;
+  };
+  Stage sg = fetch(c0);
+
+  // the wave's query blocks: fragments, and head weights w * q_scale through LDS
+  Frag a[kPfUnits][NST];
+#pragma unroll
+  for (int u = 0; u < kPfUnits; ++u) {
+    const int r = wave * RW + u / MB, h = (u % MB) * 32 + col;
+    const bool ok = r < nq && h < Hi;
+    const int64_t qh = ok ? (row0 + r) * Hi + h : row0 * Hi;
+    const uint32_t ex = FMT == kMxfp4 ? reinterpret_cast<const uint32_t*>(p.q_e8m0)[qh] : 0u;
+#pragma unroll
+    for (int st = 0; st < NST; ++st) {
+      if constexpr (FMT == kFp8) {
+        a[u][st] = load_frag<FMT, DI>(p.q + qh * RB, nullptr, st, hi);
+      } else {
+        const uint4 v = *reinterpret_cast<const uint4*>(p.q + qh * RB + 32 * st + 16 * hi);
+        a[u][st].v = v8i{(int)v.x, (int)v.y, (int)v.z, (int)v.w, 0, 0, 0, 0};
+        a[u][st].scale = static_cast<int>(ex >> (8 * hi + 16 * st)) & 0xff;
+      }
+      a[u][st] = keep_or_zero(a[u][st], ok);
+    }
+  }
+  float cw[2], cq[2];
+#pragma unroll
+  for (int k = 0; k < 2; ++k) {
+    const int r = wave * RW + (lane + 64 * k) / (32 * MB), h = (lane + 64 * k) % (32 * MB);
+    const int64_t qh = r < nq && h < Hi ? (row0 + r) * Hi + h : row0 * Hi;
+    cw[k] = p.w[qh];
+    cq[k] = FMT == kFp8 ? p.q_scale[qh] : 1.0f;
+    if (!(r < nq && h < Hi)) cw[k] = cq[k] = 0.0f;
+  }
+  asm volatile("" : : : "memory");  // the loads stay above the branch
+
+  // lane i < QB: the keys visible to row i of the workgroup
+  int visl = 0;
+  if (lane < nq) {
+    const int64_t v = (pos + 1) / p.ratio;
+    visl = v > G ? G : (v < 0 ? 0 : static_cast<int>(v));
+  }
+  int vmax = visl;
+#pragma unroll
+  for (int m = QB / 2; m >= 1; m >>= 1) {
+    const int o = __shfl_xor(vmax, m, 64);
+    vmax = o > vmax ? o : vmax;
+  }
+  vmax = __builtin_amdgcn_readfirstlane(vmax);
+  const int seen = vmax < kend ? vmax : kend;
+  const int c1 = (seen + kPfChunk - 1) / kPfChunk;  // chunks [c0, c1) hold a visible key
+
+  int done = c0 * kPfChunk;  // keys written
+  if (c0 < c1) {
+#pragma unroll
+    for (int k = 0; k < 2; ++k) coef_lds[wave][lane + 64 * k] = cw[k] * cq[k];
+    put(0, sg);
+    __syncthreads();
+    float cf[kPfUnits][16];
+#pragma unroll
+    for (int u = 0; u < kPfUnits; ++u)
+#pragma unroll
+      for (int r4 = 0; r4 < 4; ++r4) {
+        const float4 c4 = *reinterpret_cast<const float4*>(&coef_lds[wave][u * 32 + 8 * r4 + 4 * hi]);
+        cf[u][4 * r4 + 0] = c4.x;
+        cf[u][4 * r4 + 1] = c4.y;
+        cf[u][4 * r4 + 2] = c4.z;
+        cf[u][4 * r4 + 3] = c4.w;
+      }
+    sg = fetch(c0 + 1);  // (past the split's last chunk: read, never stored)
+
+    // where the lane's scores go: of row pair q, the first row from the lower half-wave and
+    // the second from the upper.  Buffer stores, which drop what lies beyond the descriptor's
+    // size: a branch around the store would end the basic block that interleaves the units.
+    float* const wout = p.scores + (row0 + wave * RW) * p.sstride;
+    const __amdgpu_buffer_rsrc_t rsrc =
+        __builtin_amdgcn_make_buffer_rsrc(wout, 0, static_cast<int>(RW * p.sstride * 4), 0x00027000);
+    uint32_t out[NP];
+    int lim[NP], vis[NP];
+#pragma unroll
+    for (int q = 0; q < NP; ++q) {
+      const int r = wave * RW + 2 * q + hi;
+      out[q] = static_cast<uint32_t>(((2 * q + hi) * p.sstride + col) * 4);
+      lim[q] = r < nq ? kend - col : 0;
+      vis[q] = __shfl(visl, r, 64) - col;
+    }
+    const float inv_sqrt_di = 1.0f / sqrt_rn(static_cast<float>(DI));
+
+    // fragment pieces of the lane's key in a tile of the buffer
+    constexpr int kFp = FMT == kFp8 ? 2 : 1;  // 16-byte pieces per step
+    const int sw = RB == 128 ? (col >> 1) & 7 : (col >> 2) & 3;
+    int fat[NST * kFp];
+#pragma unroll
+    for (int j = 0; j < NST * kFp; ++j) {
+      const int st = j / kFp, jj = j % kFp;
+      fat[j] = col * RB + (((st * 2 * kFp + hi * kFp + jj) ^ sw) << 4);
+    }
+    struct Keys {
+      v8i v[NST];
+      uint32_t x;
+    };
+    auto keys = [&](int base, int t) __attribute__((always_inline)) {
+      Keys k;
+#pragma unroll
+      for (int st = 0; st < NST; ++st) {
+        const uint4 lo = *reinterpret_cast<const uint4*>(kbuf + base + fat[st * kFp] + t * 32 * RB);
+        uint4 up = uint4{0u, 0u, 0u, 0u};
+        if constexpr (FMT == kFp8) up = *reinterpret_cast<const uint4*>(kbuf + base + fat[st * kFp + kFp - 1] + t * 32 * RB);
+        k.v[st] = v8i{(int)lo.x, (int)lo.y, (int)lo.z, (int)lo.w, (int)up.x, (int)up.y, (int)up.z, (int)up.w};
+      }
+      k.x = *reinterpret_cast<const uint32_t*>(kbuf + base + C::kKx + 4 * (t * 32 + col));
+      // MXFP4: bytes 0 and 2 are the scales of this half-wave's channel blocks
+      if constexpr (FMT == kMxfp4) k.x >>= 8 * hi;
+      return k;
+    };
+    auto unit = [&](int u, const Keys& k) __attribute__((always_inline)) {
+      v16f acc = {};
+#pragma unroll
+      for (int st = 0; st < NST; ++st) {
+        if constexpr (FMT == kFp8) {
+          acc = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(a[u][st].v, k.v[st], acc, 0, 0, 0, 127, 0, 127);
+        } else if (st == 0) {
+          acc = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(a[u][st].v, k.v[st], acc, 4, 4, 0, a[u][st].scale, 0,
+                                                                static_cast<int>(k.x));
+        } else {
+          acc = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(a[u][st].v, k.v[st], acc, 4, 4, 0, a[u][st].scale, 2,
+                                                                static_cast<int>(k.x));
         }
       }
-      continue;
-    }
-    // the wave's keys: B fragments and per-key scales (keys at or beyond G read key G-1;
-    // their score columns are never written)
-    Frag bf[kNkb][NST];
-    float ksv[kNkb];
+      return acc;
+    };
+    v16f acc[2];
+    // one tile: its unit 0 is in flight in acc[0]; `nxt` is the tile after it
+    auto tile = [&](int key0, const Keys& cur, const Keys& nxt) __attribute__((always_inline)) {
+      float part[RW];
 #pragma unroll
-    for (int t = 0; t < kNkb; ++t) {
-      const int64_t g = key0 + t * 32 + (lane & 31);
-      const int64_t gc = g < G ? g : G - 1;
+      for (int u = 0; u < kPfUnits; ++u) {
+        acc[(u + 1) & 1] = u + 1 < kPfUnits ? unit(u + 1, cur) : unit(0, nxt);
+        float s = u % MB == 0 ? 0.0f : part[u / MB];
 #pragma unroll
-      for (int st = 0; st < NST; ++st) bf[t][st] = load_frag<kFp8, DI>(kb_base + gc * DI, nullptr, st, hi);
-      ksv[t] = ks_base[gc];
-    }
-    for (int qi = 0; qi < nq; ++qi) {
-      const int64_t vis = vis_lds[qi];
-      float* out = p.scores + (b * S + s0 + qi) * p.sstride;
-      if (key0 < vis) {
-        Frag a[2][NST];
-#pragma unroll
-        for (int mb = 0; mb < 2; ++mb)
-#pragma unroll
-          for (int st = 0; st < NST; ++st) {
-            const uint4* src =
-                reinterpret_cast<const uint4*>(q_lds + (qi * 64 + mb * 32 + (lane & 31)) * kPfPitch + st * 64 + hi * 32);
-            const uint4 u = src[0], v = src[1];
-            a[mb][st].v = v8i{(int)u.x, (int)u.y, (int)u.z, (int)u.w, (int)v.x, (int)v.y, (int)v.z, (int)v.w};
-            a[mb][st].scale = 127;
-          }
-        // this lane's 16 accumulator rows of each M-block: 4 runs of 4 consecutive heads
-        float cf[2][16];
-#pragma unroll
-        for (int mb = 0; mb < 2; ++mb)
-#pragma unroll
-          for (int r4 = 0; r4 < 4; ++r4) {
-            const float4 c4 = *reinterpret_cast<const float4*>(coef_lds + qi * 64 + mb * 32 + 8 * r4 + 4 * hi);
-            cf[mb][4 * r4 + 0] = c4.x;
-            cf[mb][4 * r4 + 1] = c4.y;
-            cf[mb][4 * r4 + 2] = c4.z;
-            cf[mb][4 * r4 + 3] = c4.w;
-          }
-        // Software pipeline over the 4 key tiles: the MFMAs of tile t+1 are issued while the
-        // head sum of tile t runs (one MFMA per 16 VALU operations, about one MFMA's duration),
-        // so the matrix and vector units work at the same time; the stores come after.
-        float total[kNkb];
-        v16f acc[2][2];  // [tile parity][M-block]
-#pragma unroll
-        for (int mb = 0; mb < 2; ++mb) {
-          acc[0][mb] = v16f{};
-#pragma unroll
-          for (int st = 0; st < NST; ++st) acc[0][mb] = mma<kFp8>(a[mb][st], bf[0][st], acc[0][mb]);
-        }
-#pragma unroll
-        for (int t = 0; t < kNkb; ++t) {
-          const int cur = t & 1, nxt = cur ^ 1;
-          if (t + 1 < kNkb) {
-#pragma unroll
-            for (int mb = 0; mb < 2; ++mb) {
-              acc[nxt][mb] = v16f{};
-#pragma unroll
-              for (int st = 0; st < NST; ++st) acc[nxt][mb] = mma<kFp8>(a[mb][st], bf[t + 1][st], acc[nxt][mb]);
-            }
-          }
-          float part = 0.0f;
-#pragma unroll
-          for (int mb = 0; mb < 2; ++mb)
-#pragma unroll
-            for (int j = 0; j < 16; ++j) part = relu_fma(cf[mb][j], acc[cur][mb][j], part);
-          if (t + 1 < kNkb) {
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-              __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);   // one MFMA
-              __builtin_amdgcn_sched_group_barrier(0x002, 16, 0);  // sixteen VALU
-            }
-          }
-          total[t] = part + __shfl_xor(part, 32, 64);
-        }
-        if (lane < 32) {
-#pragma unroll
-          for (int t = 0; t < kNkb; ++t) {
-            const int64_t g = key0 + t * 32 + lane;
-            if (g < G) out[g] = g < vis ? (total[t] * inv_sqrt_di) * ksv[t] : -__builtin_huge_valf();
-          }
-        }
-      } else if (lane < 32) {
-#pragma unroll
-        for (int t = 0; t < kNkb; ++t) {
-          const int64_t g = key0 + t * 32 + lane;
-          if (g < G) out[g] = -__builtin_huge_valf();
+        for (int j = 0; j < 16; ++j) s = relu_fma(cf[u][j], acc[u & 1][j], s);
+        part[u / MB] = s;
+        if ((u + 1) % (2 * MB) == 0) {
+          // both half-waves' sums of a row pair: the first row's total in the lower half,
+          // the second's in the upper
+          const int q = u / (2 * MB);
+          const auto pr = __builtin_amdgcn_permlane32_swap(__float_as_uint(part[2 * q]), __float_as_uint(part[2 * q + 1]),
+                                                           false, false);
+          float sc = (__uint_as_float(pr[0]) + __uint_as_float(pr[1])) * inv_sqrt_di;
+          if constexpr (FMT == kFp8) sc = sc * __uint_as_float(cur.x);
+          sc = key0 < vis[q] ? sc : -__builtin_huge_valf();
+          __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(sc), rsrc, key0 < lim[q] ? out[q] + 4 * key0 : 0xffffffffu,
+                                                0, 0);
         }
       }
+    };
+
+    int cb = 0, nb = C::kBytes;  // the buffers of this chunk and of the next
+    Keys ka = keys(cb, 0), kc;
+    acc[0] = unit(0, ka);
+    for (int c = c0; c < c1; ++c) {  // one basic block: no branch inside
+      kc = keys(cb, 1);
+      tile(done, ka, kc);
+      ka = keys(cb, 2);
+      tile(done + 32, kc, ka);
+      put(nb, sg);  // (past the last chunk: put and read, never used)
+      lds_barrier();
+      sg = fetch(c + 2);
+      kc = keys(cb, 3);
+      tile(done + 64, ka, kc);
+      cb = nb;
+      nb = nb == 2 * C::kBytes ? 0 : nb + C::kBytes;
+      ka = keys(cb, 0);
+      tile(done + 96, kc, ka);
+      done += kPfChunk;
     }
   }
 
+  // the rest of the split's keys, which no row of the workgroup sees
+  for (int r = 0; r < RW; ++r) {
+    if (wave * RW + r >= nq) break;
+    float* orow = p.scores + (row0 + wave * RW + r) * p.sstride;
+    int g = done;
+    if ((reinterpret_cast<uintptr_t>(orow + g) & 15) == 0) {
+      const float inf = __builtin_huge_valf();
+      const int n4 = (kend - g) / 4 * 4;
+      for (int i = 4 * lane; i < n4; i += 256) *reinterpret_cast<float4*>(orow + g + i) = float4{-inf, -inf, -inf, -inf};
+      g += n4 > 0 ? n4 : 0;
+    }
+    for (int i = g + lane; i < kend; i += 64) orow[i] = -__builtin_huge_valf();
+  }
 }
 
 template <int FMT, int DI>
@@ -1123,6 +1228,29 @@ int resident_workgroups(int per_cu) {
     cus[dev] = n;
   }
   return per_cu * cus[dev];
+}
+
+// The prefill form from kPfPrefillMinRows rows per batch (below, a row block's keys are read
+// by too few rows to pay for the staging).  The keys are split over workgroups until the
+// launch fills the compute units at two workgroups each.
+template <int FMT>
+bool launch_prefill(const IdxParams& p, int64_t B, hipStream_t s) {
+  if (p.S < kPfPrefillMinRows || p.sstride > (int64_t(1) << 26)) return false;  // 32-bit offsets
+  const int mb = p.Hi <= 32 ? 1 : 2;
+  const int qb = kWaves * kPfUnits / mb;
+  const int64_t nrb = (p.S + qb - 1) / qb;
+  const int64_t chunks = (p.G + kPfChunk - 1) / kPfChunk;
+  const int64_t want = (resident_workgroups(2) + B * nrb - 1) / (B * nrb);
+  const int64_t per = want >= chunks ? 1 : (chunks + want - 1) / want;
+  const int64_t nsplit = (chunks + per - 1) / per;
+  const unsigned grid = static_cast<unsigned>(B * nrb * nsplit);
+  if (mb == 1)
+    indexer_prefill_kernel<FMT, 1><<<grid, kWaves * 64, 0, s>>>(p, static_cast<int>(nrb), static_cast<int>(nsplit),
+                                                                static_cast<int>(per));
+  else
+    indexer_prefill_kernel<FMT, 2><<<grid, kWaves * 64, 0, s>>>(p, static_cast<int>(nrb), static_cast<int>(nsplit),
+                                                                static_cast<int>(per));
+  return true;
 }
 
 IdxParams make_params(const uint8_t* q, const float* qs, const uint8_t* qe, const float* w, const uint8_t* k,
@@ -1198,30 +1326,8 @@ extern "C" int mzk_indexer_scores_fp8(const uint8_t* q_codes, const float* q_sca
   MZK_CHECK_ARG(Di % 64 == 0, "indexer_scores_fp8: Di must be a multiple of 64 (got %d)", Di);
   const IdxParams prm = make_params(q_codes, q_scales, nullptr, w, k_codes, k_scales, nullptr, S, Hi, G, k_batch_stride,
                                     positions, ratio, scores, score_stride);
-  if (Di == 128 && S >= kPfPrefillMinRows) {
-    // prefill: query rows stream through key tiles held in registers
-    const int64_t nqb = (S + kPfQb - 1) / kPfQb;
-    const int64_t nblocks = B * nqb;
-    MZK_CHECK_ARG(nblocks <= 0x7fffffff, "indexer_scores_fp8: %lld workgroups exceed the grid limit", (long long)nblocks);
-    // the staged query rows need more than the default dynamic-LDS limit: set once per device
-    static std::atomic<bool> attr_set[kMaxDevices] = {};  // setting it twice is harmless
-    int dev = 0;
-    if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= kMaxDevices) {
-      set_last_error("indexer_scores_fp8: no usable current device");
-      return MZK_ELAUNCH;
-    }
-    if (!attr_set[dev].load(std::memory_order_acquire)) {
-      if (hipFuncSetAttribute(reinterpret_cast<const void*>(indexer_prefill_fp8_kernel),
-                              hipFuncAttributeMaxDynamicSharedMemorySize, kPfLds) != hipSuccess) {
-        set_last_error("indexer_scores_fp8: cannot raise the prefill kernel's LDS limit to %d bytes", kPfLds);
-        return MZK_ELAUNCH;
-      }
-      attr_set[dev].store(true, std::memory_order_release);
-    }
-    indexer_prefill_fp8_kernel<<<static_cast<unsigned>(nblocks), kWaves * 64, kPfLds, as_stream(stream)>>>(prm, nqb);
-  } else {
+  if (Di != kDi || !launch_prefill<kFp8>(prm, B, as_stream(stream)))
     rc = launch<kFp8>(prm, B * S, Di, as_stream(stream));
-  }
   if (rc) return rc;
   MZK_LAUNCH_CHECK("indexer_scores_fp8");
   return MZK_OK;
@@ -1236,9 +1342,10 @@ extern "C" int mzk_indexer_scores_mxfp4(const uint8_t* q_packed, const uint8_t* 
   if (B * S == 0 || G == 0) return MZK_OK;
   MZK_CHECK_ARG(q_packed && q_e8m0 && w && k_packed && k_e8m0 && scores, "indexer_scores_mxfp4: null pointer");
   MZK_CHECK_ARG(Di % 64 == 0, "indexer_scores_mxfp4: Di must be a multiple of 64 (got %d)", Di);
-  rc = launch<kMxfp4>(make_params(q_packed, nullptr, q_e8m0, w, k_packed, nullptr, k_e8m0, S, Hi, G, k_batch_stride,
-                                  positions, ratio, scores, score_stride),
-                      B * S, Di, as_stream(stream));
+  const IdxParams prm = make_params(q_packed, nullptr, q_e8m0, w, k_packed, nullptr, k_e8m0, S, Hi, G, k_batch_stride,
+                                    positions, ratio, scores, score_stride);
+  if (Di != kDi || !launch_prefill<kMxfp4>(prm, B, as_stream(stream)))
+    rc = launch<kMxfp4>(prm, B * S, Di, as_stream(stream));
   if (rc) return rc;
   MZK_LAUNCH_CHECK("indexer_scores_mxfp4");
   return MZK_OK;

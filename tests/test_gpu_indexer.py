@@ -224,6 +224,40 @@ def test_fp8_prefill_kernel_matches_row_kernel(dev, b, s, hi, g, ratio, base):
     assert torch.equal(full, chunked)
 
 
+@pytest.mark.parametrize("fmt", ["fp8", "mxfp4"])
+@pytest.mark.parametrize("b,s,hi,g,ratio,order", [
+    (1, 64, 1, 1, 1, "last"), (1, 65, 32, 127, 1, "last"), (2, 79, 33, 129, 4, "shuffled"), (1, 100, 63, 300, 2, "last"),
+    (3, 71, 32, 257, 1, "shuffled"), (1, 64, 64, 5000, 1, "last"), (1, 1100, 64, 1000, 4, "causal"),
+    (2, 600, 8, 700, 4, "causal")])
+def test_prefill_chunks_match_row_kernel(dev, fmt, b, s, hi, g, ratio, order):
+    """The prefill form at the edges of its tiles: one key, key counts around the chunk of 128,
+    row counts around the 8 and 16 rows of a workgroup, 1 to 64 heads (one or two blocks of
+    32), keys split over many workgroups, rows at positions in any order, rows that see
+    nothing.  Bit for bit the row kernel's scores (the same rows in chunks below its row
+    threshold): the products and the order of the head sum are the same."""
+    gen = torch.Generator().manual_seed(7 * s + g)
+    q, k, w = _inputs(b, s, hi, 128, g, seed=s + g + hi)
+    pos = torch.arange(s, dtype=torch.int64).expand(b, s).clone()
+    if order == "shuffled":
+        pos = torch.randint(0, g * ratio + 3, (b, s), generator=gen)
+        pos[0, :9] = 0  # (with ratio > 1: nothing visible)
+    elif order == "last":
+        pos += max(0, g * ratio - s)
+    pos = pos.to(dev)
+    print(f"prefill scores: {fmt} B={b} S={s} Hi={hi} G={g} ratio={ratio} {order}", flush=True)
+    if fmt == "fp8":
+        qo, ko = MQ.quant_fp8_block(q.to(dev), 128), MQ.quant_fp8_block(k.to(dev), 128)
+        qo, ko = (qo[0], qo[1][..., 0].contiguous()), (ko[0], ko[1][..., 0].contiguous())
+        fn = MI.scores_fp8
+    else:
+        qo, ko, fn = MQ.quant_mxfp4(q.to(dev)), MQ.quant_mxfp4(k.to(dev)), MI.scores_mxfp4
+    w = w.to(dev)
+    full = fn(*qo, w, *ko, compress_ratio=ratio, positions=pos)
+    parts = [fn(*(t[:, c:c + 48] for t in qo), w[:, c:c + 48], *ko, compress_ratio=ratio, positions=pos[:, c:c + 48])
+             for c in range(0, s, 48)]
+    assert torch.equal(full, torch.cat(parts, 1))
+
+
 def test_fp8_quantizer_feeds_scores(dev):
     """GPU quantizer -> GPU scores equals oracle quantizer -> oracle scores."""
     q, k, w = _inputs(4, 1, 64, 128, 2048, seed=3)
