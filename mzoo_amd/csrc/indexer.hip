@@ -1231,12 +1231,18 @@ int resident_workgroups(int per_cu) {
 }
 
 // The prefill form from kPfPrefillMinRows rows per batch (below, a row block's keys are read
-// by too few rows to pay for the staging).  The keys are split over workgroups until the
-// launch fills the compute units at two workgroups each.
+// by too few rows to pay for the staging), unless the row form's workgroups are all resident
+// at once, two per compute unit up to 32 heads and one above: its start (query, first chunk,
+// barrier) takes 1.5 to 2 us longer than a row workgroup's (MXFP4, row -> prefill form: 64
+// rows x 516 keys 3.7 -> 5.1 us at 32 heads and 4.4 -> 4.7 us at 64; 8 x 64 rows x 141 keys
+// 4.3 -> 5.1 and 5.1 -> 4.7; 100 rows x 3025 keys 5.6 -> 5.3 and 7.0 -> 6.1; 64 x 64 rows x 32
+// keys 9.6 -> 5.2 and 12.8 -> 6.1; 8000 rows x 5000 keys 268 -> 109 and 405 -> 167).  The keys
+// are split over workgroups until the launch fills the compute units at two workgroups each.
 template <int FMT>
 bool launch_prefill(const IdxParams& p, int64_t B, hipStream_t s) {
   if (p.S < kPfPrefillMinRows || p.sstride > (int64_t(1) << 26)) return false;  // 32-bit offsets
   const int mb = p.Hi <= 32 ? 1 : 2;
+  if (B * p.S * ((p.G + kKeysPerWg - 1) / kKeysPerWg) <= resident_workgroups(mb == 1 ? 2 : 1)) return false;
   const int qb = kWaves * kPfUnits / mb;
   const int64_t nrb = (p.S + qb - 1) / qb;
   const int64_t chunks = (p.G + kPfChunk - 1) / kPfChunk;

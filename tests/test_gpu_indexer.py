@@ -226,11 +226,12 @@ def test_fp8_prefill_kernel_matches_row_kernel(dev, b, s, hi, g, ratio, base):
 
 @pytest.mark.parametrize("fmt", ["fp8", "mxfp4"])
 @pytest.mark.parametrize("b,s,hi,g,ratio,order", [
-    (1, 64, 1, 1, 1, "last"), (1, 65, 32, 127, 1, "last"), (2, 79, 33, 129, 4, "shuffled"), (1, 100, 63, 300, 2, "last"),
-    (3, 71, 32, 257, 1, "shuffled"), (1, 64, 64, 5000, 1, "last"), (1, 1100, 64, 1000, 4, "causal"),
-    (2, 600, 8, 700, 4, "causal")])
+    (2, 35000, 1, 1, 1, "last"), (33, 65, 32, 127, 1, "last"), (7, 79, 33, 129, 4, "shuffled"), (1, 300, 63, 300, 2, "last"),
+    (17, 71, 32, 257, 1, "shuffled"), (1, 64, 64, 5000, 1, "last"), (1, 1100, 64, 1000, 4, "causal"),
+    (2, 600, 8, 700, 4, "causal"), (1, 64, 32, 4096, 1, "last"), (1, 64, 32, 4097, 1, "last")])
 def test_prefill_chunks_match_row_kernel(dev, fmt, b, s, hi, g, ratio, order):
-    """The prefill form at the edges of its tiles: one key, key counts around the chunk of 128,
+    """The prefill form at the edges of its tiles: one key (more rows than the row form takes),
+    the line between the forms (512 row workgroups), key counts around the chunk of 128,
     row counts around the 8 and 16 rows of a workgroup, 1 to 64 heads (one or two blocks of
     32), keys split over many workgroups, rows at positions in any order, rows that see
     nothing.  Bit for bit the row kernel's scores (the same rows in chunks below its row
@@ -254,8 +255,9 @@ def test_prefill_chunks_match_row_kernel(dev, fmt, b, s, hi, g, ratio, order):
     w = w.to(dev)
     full = fn(*qo, w, *ko, compress_ratio=ratio, positions=pos)
     parts = [fn(*(t[:, c:c + 48] for t in qo), w[:, c:c + 48], *ko, compress_ratio=ratio, positions=pos[:, c:c + 48])
-             for c in range(0, s, 48)]
-    assert torch.equal(full, torch.cat(parts, 1))
+             for c in (range(0, s, 48) if b * s <= 65535 else [0, s - 48])]
+    got = full if b * s <= 65535 else torch.cat([full[:, :48], full[:, -48:]], 1)
+    assert torch.equal(got, torch.cat(parts, 1))
 
 
 def test_fp8_quantizer_feeds_scores(dev):
