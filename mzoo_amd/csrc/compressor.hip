@@ -16,15 +16,43 @@
 //   pooled: sum from 0 in r order of kv_r * p_r;
 //   RMSNorm: lane l of the wave sums channels l, l+64, ... in order from 0, then the xor
 //   butterfly (32, 16, 8, 4, 2, 1); var = sum / D; rsqrt = 1 / sqrt (correctly rounded).
-// Layout: one wave per (b, group); lane l owns channels l + 64 i (coalesced 256 B rows).
+// Layout: one wave per (b, group), lane l owning channels l + 64 i (coalesced 256 B rows), or
+// one workgroup per group where the ratio is large.
 #include "common.h"
 
 namespace mzk {
 namespace {
 
 constexpr int kMaxPerLane = 16;  // D <= 1024
+constexpr int kPoolAhead = 2;    // channels per lane loaded together (2 * ratio registers each)
 
-template <int ODT, int WDT>
+// The pooled value of one channel over R tokens held in registers: the operations and order
+// above; exp(g_r - max) is formed once and used in the sum and in the weight.
+template <int R>
+__device__ __forceinline__ float pool_channel(const float (&k)[R], const float (&g)[R]) {
+  float m = g[0];
+#pragma unroll
+  for (int r = 1; r < R; ++r) m = fmaxf(m, g[r]);
+  float e[R];
+  float s = 0.0f;
+#pragma unroll
+  for (int r = 0; r < R; ++r) {
+    e[r] = exp_pinned(g[r] - m);
+    s = s + e[r];
+  }
+  float acc = 0.0f;
+#pragma unroll
+  for (int r = 0; r < R; ++r) acc = acc + k[r] * div_rn(e[r], s);
+  return acc;
+}
+
+// Ratios 1, 2 and 4: one wave per group, kPoolAhead channels' whole groups loaded into
+// registers before the first is used.  It was bound by latency -- loops that read each gate
+// three times from the cache, one load in flight, and formed each exp twice; now by the
+// divisions and exps (some 55 operations per token and channel), about twice its memory time.
+// 8192 tokens x 576 channels: ratio 4 35.9 -> 14.0 us, ratio 2 24.3 -> 13.6 us (4 channels
+// ahead 14.2, 8 15.3, 16 15.4).
+template <int ODT, int WDT, int RATIO>
 __global__ void __launch_bounds__(256) compress_kernel(const float* __restrict__ kv, const float* __restrict__ gate,
                                                        int64_t B, int64_t n_groups, int ratio, int D,
                                                        int64_t tokens_per_batch, const void* __restrict__ weight,
@@ -39,29 +67,36 @@ __global__ void __launch_bounds__(256) compress_kernel(const float* __restrict__
 
   float h[kMaxPerLane];
   float ss = 0.0f;
+  constexpr int R = RATIO, A = kPoolAhead;
+  static_assert(kMaxPerLane % A == 0, "whole batches of channels");
 #pragma unroll
-  for (int i = 0; i < kMaxPerLane; ++i) {
-    const int d = lane + 64 * i;
-    h[i] = 0.0f;
-    if (d < D) {
-      float v;
-      if (ratio == 1) {
-        v = kvb[d];
-      } else {
-        float m = gtb[d];
-        for (int r = 1; r < ratio; ++r) m = fmaxf(m, gtb[static_cast<int64_t>(r) * D + d]);
-        float s = 0.0f;
-        for (int r = 0; r < ratio; ++r) s = s + exp_pinned(gtb[static_cast<int64_t>(r) * D + d] - m);
-        float acc = 0.0f;
-        for (int r = 0; r < ratio; ++r) {
-          const float e = exp_pinned(gtb[static_cast<int64_t>(r) * D + d] - m);
-          acc = acc + kvb[static_cast<int64_t>(r) * D + d] * div_rn(e, s);
+  for (int i0 = 0; i0 < kMaxPerLane; i0 += A) {
+    if (64 * i0 < D) {  // uniform
+      float k[A][R], g[A][R];
+#pragma unroll
+      for (int a = 0; a < A; ++a) {
+        // channels at or beyond D read channel D - 1 and are dropped
+        const int d = lane + 64 * (i0 + a) < D ? lane + 64 * (i0 + a) : D - 1;
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+          k[a][r] = kvb[r * D + d];
+          g[a][r] = R > 1 ? gtb[r * D + d] : 0.0f;
         }
-        v = acc;
       }
-      v = round_to_dtype<ODT>(v);  // latent.to(dtype) before the norm
-      h[i] = v;
-      ss = ss + v * v;
+#pragma unroll
+      for (int a = 0; a < A; ++a) {
+        h[i0 + a] = 0.0f;
+        if (64 * (i0 + a) < D) {  // uniform
+          const float v = round_to_dtype<ODT>(R > 1 ? pool_channel<R>(k[a], g[a]) : k[a][0]);
+          if (lane + 64 * (i0 + a) < D) {
+            h[i0 + a] = v;
+            ss = ss + v * v;
+          }
+        }
+      }
+    } else {
+#pragma unroll
+      for (int a = 0; a < A; ++a) h[i0 + a] = 0.0f;
     }
   }
   // xor butterfly: every lane ends with the same total
@@ -77,6 +112,72 @@ __global__ void __launch_bounds__(256) compress_kernel(const float* __restrict__
       const float w = load_as_f32<WDT>(weight, d);
       store_from_f32<ODT>(out, rid * D + d, w * normed);
     }
+  }
+}
+
+// Any other ratio: one workgroup per group, thread d owns channel d and walks the group's
+// tokens in order, kTokensAhead of them loaded together; the channels meet in LDS, where wave
+// 0 sums their squares in the pinned order.  A group of 128 tokens in one wave took 9 channels
+// x 128 tokens x 3 dependent reads per lane in turn: 8192 tokens x 576 channels at ratio 128
+// 889 -> 62.8 us, at ratio 8 59 -> 14.5, at ratio 3 30 -> 24 (16 tokens ahead: 59.5, 23.6 and
+// 41.5 us; 4: 72, 16.1 and 19.4).
+constexpr int kTokensAhead = 8;
+
+template <int ODT, int WDT>
+__global__ void __launch_bounds__(64 * kMaxPerLane)
+    compress_wide_kernel(const float* __restrict__ kv, const float* __restrict__ gate, int64_t n_groups, int ratio, int D,
+                         int64_t tokens_per_batch, const void* __restrict__ weight, float eps, void* __restrict__ out) {
+  __shared__ float h_lds[64 * kMaxPerLane];
+  __shared__ float inv_lds;
+  const int64_t rid = blockIdx.x;
+  const int64_t b = rid / n_groups;
+  const int64_t g = rid - b * n_groups;
+  const int d = threadIdx.x < D ? threadIdx.x : D - 1;  // (threads beyond D: a channel again, dropped)
+  const float* k = kv + (b * tokens_per_batch + g * ratio) * D + d;
+  const float* gt = gate + (b * tokens_per_batch + g * ratio) * D + d;
+  // the group's next tokens (at or beyond its end the last one, not used)
+  auto ahead = [&](const float* p, int r0, float (&v)[kTokensAhead]) __attribute__((always_inline)) {
+#pragma unroll
+    for (int j = 0; j < kTokensAhead; ++j) v[j] = p[static_cast<int64_t>(r0 + j < ratio ? r0 + j : ratio - 1) * D];
+  };
+  float gv[kTokensAhead], kvv[kTokensAhead];
+  float m = gt[0];
+  for (int r0 = 0; r0 < ratio; r0 += kTokensAhead) {
+    ahead(gt, r0, gv);
+#pragma unroll
+    for (int j = 0; j < kTokensAhead; ++j)
+      if (r0 + j > 0 && r0 + j < ratio) m = fmaxf(m, gv[j]);
+  }
+  float s = 0.0f;
+  for (int r0 = 0; r0 < ratio; r0 += kTokensAhead) {
+    ahead(gt, r0, gv);
+#pragma unroll
+    for (int j = 0; j < kTokensAhead; ++j)
+      if (r0 + j < ratio) s = s + exp_pinned(gv[j] - m);
+  }
+  float acc = 0.0f;
+  for (int r0 = 0; r0 < ratio; r0 += kTokensAhead) {
+    ahead(gt, r0, gv);
+    ahead(k, r0, kvv);
+#pragma unroll
+    for (int j = 0; j < kTokensAhead; ++j)
+      if (r0 + j < ratio) acc = acc + kvv[j] * div_rn(exp_pinned(gv[j] - m), s);
+  }
+  const float v = round_to_dtype<ODT>(acc);  // latent.to(dtype) before the norm
+  h_lds[threadIdx.x] = v;
+  __syncthreads();
+  if (threadIdx.x < 64) {
+    float ss = 0.0f;
+    for (int c = threadIdx.x; c < D; c += 64) ss = ss + h_lds[c] * h_lds[c];
+#pragma unroll
+    for (int x = 32; x >= 1; x >>= 1) ss = ss + __shfl_xor(ss, x, 64);
+    const float var = div_rn(ss, static_cast<float>(D));
+    if (threadIdx.x == 0) inv_lds = div_rn(1.0f, sqrt_rn(var + eps));
+  }
+  __syncthreads();
+  if (threadIdx.x < D) {
+    const float normed = round_to_dtype<ODT>(v * inv_lds);
+    store_from_f32<ODT>(out, rid * D + d, load_as_f32<WDT>(weight, d) * normed);
   }
 }
 
@@ -157,14 +258,27 @@ __global__ void rope_kernel(const void* __restrict__ x, const float* __restrict_
   store_from_f32<DT>(y, base + (D - rd) + 2 * i + 1, ev * s + od * c);
 }
 
+template <int ODT, int WDT>
+void launch_compress_r(const float* kv, const float* gate, int64_t B, int64_t n, int ratio, int D, int64_t tpb,
+                       const void* w, float eps, void* out, hipStream_t s) {
+  const unsigned grid = static_cast<unsigned>((B * n + 3) / 4);
+  switch (ratio) {
+    case 1: compress_kernel<ODT, WDT, 1><<<grid, 256, 0, s>>>(kv, gate, B, n, ratio, D, tpb, w, eps, out); break;
+    case 2: compress_kernel<ODT, WDT, 2><<<grid, 256, 0, s>>>(kv, gate, B, n, ratio, D, tpb, w, eps, out); break;
+    case 4: compress_kernel<ODT, WDT, 4><<<grid, 256, 0, s>>>(kv, gate, B, n, ratio, D, tpb, w, eps, out); break;
+    default:
+      compress_wide_kernel<ODT, WDT><<<static_cast<unsigned>(B * n), (D + 63) / 64 * 64, 0, s>>>(kv, gate, n, ratio, D, tpb,
+                                                                                               w, eps, out);
+  }
+}
+
 template <int ODT>
 int launch_compress_w(int wdt, const float* kv, const float* gate, int64_t B, int64_t n, int ratio, int D, int64_t tpb,
                       const void* w, float eps, void* out, hipStream_t s) {
-  const unsigned grid = static_cast<unsigned>((B * n + 3) / 4);
   switch (wdt) {
-    case MZK_F32: compress_kernel<ODT, MZK_F32><<<grid, 256, 0, s>>>(kv, gate, B, n, ratio, D, tpb, w, eps, out); break;
-    case MZK_BF16: compress_kernel<ODT, MZK_BF16><<<grid, 256, 0, s>>>(kv, gate, B, n, ratio, D, tpb, w, eps, out); break;
-    case MZK_F16: compress_kernel<ODT, MZK_F16><<<grid, 256, 0, s>>>(kv, gate, B, n, ratio, D, tpb, w, eps, out); break;
+    case MZK_F32: launch_compress_r<ODT, MZK_F32>(kv, gate, B, n, ratio, D, tpb, w, eps, out, s); break;
+    case MZK_BF16: launch_compress_r<ODT, MZK_BF16>(kv, gate, B, n, ratio, D, tpb, w, eps, out, s); break;
+    case MZK_F16: launch_compress_r<ODT, MZK_F16>(kv, gate, B, n, ratio, D, tpb, w, eps, out, s); break;
     default: set_last_error("compress: unsupported weight dtype %d", wdt); return MZK_EINVAL;
   }
   return MZK_OK;

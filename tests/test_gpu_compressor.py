@@ -40,6 +40,25 @@ def test_compress_bit_exact(dev, dtype, ratio, d):
     assert np.array_equal(_bits(got), _obits(want, dtype))
 
 
+@pytest.mark.parametrize("ratio,d", [(2, 1), (4, 65), (4, 1024), (2, 1000), (1, 129), (3, 100), (7, 1024), (8, 576),
+                                     (9, 64), (130, 1), (17, 65)])
+def test_compress_edges_bit_exact(dev, ratio, d):
+    """Channel counts around the wave and the two channels a lane loads together (ratios 1, 2,
+    4), token counts around the 8 that the other ratios load together; a gate of -inf and one
+    far below the maximum take their weights' limits."""
+    gen = torch.Generator().manual_seed(ratio * 1000 + d)
+    b, n = 2, 5
+    kv = torch.randn(b, n * ratio + 1, d, generator=gen)
+    gate = torch.randn(b, n * ratio + 1, d, generator=gen) * 30
+    if ratio > 1:
+        gate[0, 1, d // 2] = float("-inf")
+        gate[1, 0, 0] = -200.0
+    w = (1 + 0.1 * torch.randn(d, generator=gen)).bfloat16()
+    got = MC.compress(kv.to(dev), gate.to(dev) if ratio > 1 else None, ratio, w.to(dev), 1e-20, torch.bfloat16, n_groups=n)
+    want = C.compress(kv[:, :n * ratio].numpy(), gate[:, :n * ratio].numpy(), ratio, w.float().numpy(), 1e-20, "bfloat16")
+    assert np.array_equal(_bits(got), _obits(want, torch.bfloat16))
+
+
 def test_compressor_carry_matches_one_shot(dev):
     gen = torch.Generator().manual_seed(9)
     kv = torch.randn(2, 37, 576, generator=gen).to(dev)
