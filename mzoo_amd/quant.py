@@ -60,15 +60,28 @@ def _fake_quant_fp4_block(x: torch.Tensor, block_size: int, e4m3_scales: bool = 
     return y.view(x.shape)
 
 
-def quant_fp8_block(x: torch.Tensor, block_size: int = 128) -> tuple[torch.Tensor, torch.Tensor]:
-    """x [..., n] -> (codes uint8 [..., n], scales fp32 [..., n/block_size])."""
+def _take_out(out, want) -> tuple[torch.Tensor, torch.Tensor]:
+    """``out`` as the contiguous tensors of the wanted (shape, dtype) pairs on one device, or
+    new ones."""
+    (device, *specs) = want
+    if out is None:
+        return tuple(torch.empty(shape, dtype=dt, device=device) for shape, dt in specs)
+    for t, (shape, dt) in zip(out, specs):
+        if tuple(t.shape) != tuple(shape) or t.dtype != dt or t.device != device or not t.is_contiguous():
+            raise ValueError(f"out: contiguous {dt} {tuple(shape)} on {device} expected, got {t.dtype} {tuple(t.shape)}")
+    return tuple(out)
+
+
+def quant_fp8_block(x: torch.Tensor, block_size: int = 128, out=None) -> tuple[torch.Tensor, torch.Tensor]:
+    """x [..., n] -> (codes uint8 [..., n], scales fp32 [..., n/block_size]); into the two
+    contiguous tensors ``out`` if given."""
     _lib.require_gpu(x)
     n = x.shape[-1]
     if n % block_size:
         raise ValueError(f"quant_fp8_block: n={n} is not a multiple of block_size={block_size}")
     xc = x.contiguous()
-    codes = torch.empty(x.shape, dtype=torch.uint8, device=x.device)
-    scales = torch.empty(*x.shape[:-1], n // block_size, dtype=torch.float32, device=x.device)
+    codes, scales = _take_out(out, (x.device, (x.shape, torch.uint8),
+                                    ((*x.shape[:-1], n // block_size), torch.float32)))
     _lib.call("mzk_quant_fp8_block", xc.data_ptr(), _lib.dtype_code(x.dtype), _rows(xc), n, block_size,
               codes.data_ptr(), scales.data_ptr(), _lib.stream_of(x))
     return codes, scales
@@ -85,16 +98,16 @@ def dequant_fp8_block(codes: torch.Tensor, scales: torch.Tensor, block_size: int
     return y
 
 
-def quant_mxfp4(x: torch.Tensor) -> tuple[torch.Tensor, torch.Tensor]:
+def quant_mxfp4(x: torch.Tensor, out=None) -> tuple[torch.Tensor, torch.Tensor]:
     """x [..., n] -> (packed uint8 [..., n/2], e8m0 uint8 [..., n/32]) of
-    ``_fake_quant_fp4_block(x, 32)``."""
+    ``_fake_quant_fp4_block(x, 32)``; into the two contiguous tensors ``out`` if given."""
     _lib.require_gpu(x)
     n = x.shape[-1]
     if n % 32:
         raise ValueError(f"quant_mxfp4: n={n} is not a multiple of 32")
     xc = x.contiguous()
-    packed = torch.empty(*x.shape[:-1], n // 2, dtype=torch.uint8, device=x.device)
-    e8m0 = torch.empty(*x.shape[:-1], n // 32, dtype=torch.uint8, device=x.device)
+    packed, e8m0 = _take_out(out, (x.device, ((*x.shape[:-1], n // 2), torch.uint8),
+                                   ((*x.shape[:-1], n // 32), torch.uint8)))
     _lib.call("mzk_quant_mxfp4", xc.data_ptr(), _lib.dtype_code(x.dtype), _rows(xc), n, packed.data_ptr(),
               e8m0.data_ptr(), _lib.stream_of(x))
     return packed, e8m0
