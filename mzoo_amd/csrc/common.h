@@ -342,9 +342,10 @@ __device__ __forceinline__ float lane_xor(float v) {
 }
 
 // Maximum of values >= 0 or NaN (NaN wins, see nn_max) over aligned groups of `group`
-// consecutive lanes (a power of two <= 32), by exact xor-partner exchanges; every lane of a
+// consecutive lanes (a power of two <= 64), by exact xor-partner exchanges; every lane of a
 // group ends with the group's maximum.
 __device__ __forceinline__ float group_max(float v, int group) {
+  if (group > 32) v = nn_max(v, lane_xor<32>(v));
   if (group > 16) v = nn_max(v, lane_xor<16>(v));
   if (group > 8) v = nn_max(v, lane_xor<8>(v));
   if (group > 4) v = nn_max(v, lane_xor<4>(v));

@@ -186,3 +186,14 @@ def test_pack_cache_v41_bit_exact(dev, fmt, d, dtype):
     dst = torch.randperm(64, generator=gen)[:37]
     MQ.pack_cache_v41(x.to(dev), fmt, out=cache, dst_index=dst)
     assert torch.equal(cache[dst.to(dev)], got)
+
+
+@pytest.mark.parametrize("bs", [4, 16, 64, 128, 256])
+def test_fp8_block_sizes_match_oracle(dev, bs):
+    """Every block size the quantizer takes has one scale per whole block (a block of 256 fills
+    a wave; each block's maximum sits in its second half)."""
+    x = torch.randn(5, 512, generator=torch.Generator().manual_seed(bs))
+    x.view(-1, bs)[:, -1] = 300.0
+    codes, scales = MQ.quant_fp8_block(x.to(dev), bs)
+    wc, ws = Q.fp8_block_codes(x.numpy(), bs)
+    assert np.array_equal(codes.cpu().numpy(), wc.reshape(5, 512)) and np.array_equal(scales.cpu().numpy(), ws.reshape(5, -1))
