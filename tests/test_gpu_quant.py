@@ -197,3 +197,31 @@ def test_fp8_block_sizes_match_oracle(dev, bs):
     codes, scales = MQ.quant_fp8_block(x.to(dev), bs)
     wc, ws = Q.fp8_block_codes(x.numpy(), bs)
     assert np.array_equal(codes.cpu().numpy(), wc.reshape(5, 512)) and np.array_equal(scales.cpu().numpy(), ws.reshape(5, -1))
+
+
+@pytest.mark.parametrize("bs,n", [(16, 48), (32, 160), (64, 64), (128, 128), (128, 640), (256, 512)])
+def test_fp8_wide_form_matches_narrow(dev, bs, n):
+    """From 2^21 bf16 elements the FP8 quantizer takes 16 per thread: codes and scale bits equal
+    the narrow form's (the same rows in parts below that size, and an operand that is not
+    16-byte aligned), over random bit patterns -- every magnitude, subnormals, signed zeros --
+    and blocks that hold infinities or NaNs; the last workgroup is ragged."""
+    rows = -(-(1 << 21) // n) + 3
+    gen = torch.Generator().manual_seed(bs + n)
+    bits = torch.randint(-32768, 32768, (rows, n), generator=gen, dtype=torch.int32).to(torch.int16)
+    special = (bits & 0x7F80) == 0x7F80
+    bits = torch.where(special, bits & ~0x4000, bits)  # finite, then planted non-finite values
+    scale = torch.randint(0, 4, (rows, 1), generator=gen)
+    bits = torch.where(scale == 0, (bits & 0x807F) | 0x3F80, bits)  # rows of one binade: ties
+    for i, v in enumerate((0x7F80, -128, 0x7FC0, -64)):  # inf, -inf, nan, -nan
+        bits[5 + i, (7 * i) % n] = v
+    bits[11] = 0
+    x = bits.view(torch.bfloat16).to(dev)
+    codes, scales = MQ.quant_fp8_block(x, bs)
+    half = rows // 2
+    for a, z in ((0, half), (half, rows)):
+        c, s = MQ.quant_fp8_block(x[a:z], bs)
+        assert torch.equal(codes[a:z], c) and torch.equal(scales[a:z].view(torch.int32), s.view(torch.int32))
+    buf = torch.empty(x.numel() + 1, dtype=torch.bfloat16, device=dev)
+    buf[1:] = x.view(-1)
+    c, s = MQ.quant_fp8_block(buf[1:].view(rows, n), bs)
+    assert torch.equal(codes, c) and torch.equal(scales.view(torch.int32), s.view(torch.int32))
