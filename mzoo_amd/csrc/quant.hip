@@ -126,8 +126,8 @@ __device__ __forceinline__ void quant_fp8_16(const uint16_t* __restrict__ x, uin
 
 // What bounds quant_fp8_block_kernel is its 24.5 vector operations per element (64-bit
 // indices, clamps and one scale per four elements): 524288 x 128 bf16, 46 us.  This form takes
-// about 4 and runs at the memory's pace: 23 us, 8.7 TB/s of its 201 MB (held by the
-// last-level cache between runs).
+// about 4 and runs at the memory's pace: 29 us, 6.9 TB/s of its 201 MB (partly held by the
+// last-level cache).
 __global__ void __launch_bounds__(256)
     quant_fp8_wide_kernel(const uint16_t* __restrict__ x, uint8_t* __restrict__ codes, float* __restrict__ scales,
                           int64_t nthreads, int group) {
@@ -369,8 +369,9 @@ void launch_fake(const void* x, void* y, int64_t rows, int64_t n, int bs, bool f
 template <int DT>
 void launch_quant_fp8(const void* x, int64_t rows, int64_t n, int bs, uint8_t* codes, float* scales, hipStream_t s) {
   // the wide form: bf16 with 16-byte aligned operands, blocks of whole threads (16 elements) in
-  // one wave, and enough threads for two waves on every SIMD (131072 on 256 compute units); below
-  // that both take a few microseconds, most of it the launch
+  // one wave, from 2^21 elements, which give every SIMD two of its waves (narrow -> wide form:
+  // 2^21 elements 3.4 -> 2.7 us, 2^22 4.8 -> 3.3, 2^24 14.2 -> 9.4, 2^26 45.8 -> 29.0); below,
+  // both take the launch's 2.4 to 2.8 us
   if constexpr (DT == MZK_BF16) {
     if (pow2_in(bs, 16, 256) && aligned16(x) && aligned16(codes) && rows * n / 16 >= 131072) {
       const int64_t wide = rows * n / 16;
