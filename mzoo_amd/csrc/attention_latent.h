@@ -21,11 +21,15 @@
 // 2050 cycles (bf16; fp8 2280): one wave per SIMD issues an instruction every 5 cycles or so,
 // 250 of them a tile, and the barrier adds 180; deeper operand prefetch changed nothing.
 //
-// Softmax: the exponent's reference is fixed, 2^32 above the first tile's maximum: softmax is
-// exact for any reference as long as nothing overflows or underflows, and this one leaves the
-// true maximum 122 powers of two of room above the first tile's, and everything 2^-94 below
-// it a normal number.  A score beyond that makes the workgroup start again from the true maxima of a
-// pass over the scores alone.  So no tile waits for the other waves' maxima, and O^T is never rescaled.
+// Softmax: the exponent's reference is fixed at the first tile's maximum: softmax is exact for
+// any reference as long as nothing overflows or underflows.  The weights that count are then
+// 1 or more (the true maximum is no lower), so no value of an entry is lost at the low
+// end.  At the high end a weight reaches 2^(rise of the scores above the first tile), which
+// multiplies an entry's value: up to 2^kRoomNear that is the range of a softmax rescaled as it goes;
+// above, the accumulators are looked at after the pass, and above 2^kRoomAbove the row sum itself
+// would overflow.  Where either overflowed, the workgroup starts again from the true maxima of
+// a pass over the scores alone (weights at most 1).  So no tile waits for the other waves'
+// maxima, and O^T is never rescaled.
 
 // An entry's table code: its source in the top two bits, its index below them.
 constexpr uint32_t kEmptyEntry = 0xffffffffu;
@@ -41,7 +45,7 @@ struct LatentSmem {
   static constexpr int MASK = TAB + 4 * TABN;  // valid entries of each tile
   static constexpr int PMAX = MASK + 4 * (TABN / kTile + 5);  // [2 eh][64]; 16-byte aligned
   static constexpr int LSUM = PMAX + 512;      // [2 eh][64]
-  static constexpr int RED = LSUM + 512;       // reduction scratch, redo
+  static constexpr int RED = LSUM + 512;       // reduction scratch, redo, high
   static constexpr int LDS = RED + 64;
 };
 
@@ -52,7 +56,7 @@ struct LatentSmem {
 // and the transposing reads of V^T.
 __device__ __forceinline__ int lat_swz(int e) { return e & 7; }
 
-constexpr float kRoomBelow = 32.0f, kRoomAbove = 90.0f;  // log2 units around the reference
+constexpr float kRoomNear = kLazy, kRoomAbove = 100.0f;    // log2 units above the reference
 constexpr float kMasked = -3.0e38f;                        // a masked entry's score: weight 0
 
 // A tile in flight: one thread's pieces of entry tid / 8.
@@ -77,6 +81,7 @@ sparse_mqa_latent_kernel(const AttnParams p) {
   float* const lsum = reinterpret_cast<float*>(smem + M::LSUM);
   int* const wred = reinterpret_cast<int*>(smem + M::RED);
   int* const redo = wred + 8;
+  int* const high = wred + 9;
 
   const int tid = threadIdx.x;
   const int lane = tid & 63;
@@ -140,7 +145,7 @@ sparse_mqa_latent_kernel(const AttnParams p) {
       __hip_atomic_fetch_add(reinterpret_cast<uint64_t*>(mrec), 1ull << (8 * xcc_id()), __ATOMIC_RELAXED,
                              __HIP_MEMORY_SCOPE_AGENT);
   }
-  if (tid == 0) *redo = 0;
+  if (tid == 0) *redo = *high = 0;
 
   // ---- the split's entry table -----------------------------------------------------------
   int32_t* const sidx = reinterpret_cast<int32_t*>(smem);  // the row's list, where tiles come later
@@ -396,12 +401,8 @@ sparse_mqa_latent_kernel(const AttnParams p) {
         agree_max(max4(v[0]), max4(v[1]));
         // a head without a finite score in its first tile (or with NaN): from the true maxima
 #pragma unroll
-        for (int hg = 0; hg < 4; ++hg) {
+        for (int hg = 0; hg < 4; ++hg)
           if (!(m4[hg] > -__builtin_huge_valf())) *redo = 1;
-          m4[hg] = m4[hg] + kRoomBelow;
-        }
-        m_own[0] = m_own[0] + kRoomBelow;
-        m_own[1] = m_own[1] + kRoomBelow;
       }
       // the raw scores' maxima, for the check at the end (-inf where masked: the first tile's)
       m_seen[0] = m_seen[1] = -__builtin_huge_valf();
@@ -551,8 +552,11 @@ sparse_mqa_latent_kernel(const AttnParams p) {
           if (hg == 0 && i + VH < NI) read_v(vt, i + VH, va[(i + VH) % (VH + 1)]);
         });
     }
-    if (!given && (m_seen[0] * p.scale_log2 > m_own[0] + kRoomAbove || m_seen[1] * p.scale_log2 > m_own[1] + kRoomAbove))
-      *redo = 1;
+    if (!given) {
+      const float rise = fmaxf(m_seen[0] * p.scale_log2 - m_own[0], m_seen[1] * p.scale_log2 - m_own[1]);
+      if (rise > kRoomNear) *high = 1;
+      if (rise > kRoomAbove) *redo = 1;
+    }
   };
 
   // the true maxima of every head over the split (m4 / m_own): scores only
@@ -643,9 +647,8 @@ sparse_mqa_latent_kernel(const AttnParams p) {
         asm volatile("" : "+a"(x));
         qf[st][b] = __builtin_bit_cast(v8bf, x);
       }
-#pragma unroll 1
-    for (int attempt = 0; attempt < 2; ++attempt) {
-      pass(attempt != 0);
+    for (bool given = false;; given = true) {
+      pass(given);
       // each head's row sum: its four lanes, then the two entry halves
 #pragma unroll
       for (int b = 0; b < 2; ++b) {
@@ -656,7 +659,28 @@ sparse_mqa_latent_kernel(const AttnParams p) {
       lds_barrier();
 #pragma unroll
       for (int hg = 0; hg < 4; ++hg) l4[hg] = lsum[16 * hg + e16] + lsum[64 + 16 * hg + e16];
-      if (attempt != 0 || *redo == 0) break;  // uniform: set before the barrier above
+      if (__builtin_expect(!given && *high != 0, 0)) {  // uniform: set before the barrier above
+        // O^T through the tiles' place, half of it at a time, each lane its own: a few stores
+        // and a short loop.  Looked at in registers it took 3.6 KB of code, and a decode step
+        // (whose kernel runs from a cold instruction cache) 1 us whether or not it was entered.
+        float any_bad = 0.0f;  // NaN if an accumulator is not finite
+        v4f* const slot = reinterpret_cast<v4f*>(smem) + tid;
+        static_assert(2 * NI * NT * 16 <= M::PB, "half of O^T in the tiles' place");
+#pragma unroll
+        for (int half = 0; half < 2; ++half) {
+#pragma unroll
+          for (int k = 0; k < 2 * NI; ++k) slot[k * NT] = acc[k >> 1][2 * half + (k & 1)];
+#pragma unroll 1
+          for (int k = 0; k < 2 * NI; ++k) {
+            const v4f x = slot[k * NT];
+#pragma unroll
+            for (int r = 0; r < 4; ++r) any_bad = __builtin_fmaf(x[r], 0.0f, any_bad);
+          }
+        }
+        if (any_bad != 0.0f) *redo = 1;
+        lds_barrier();
+      }
+      if (given || *redo == 0) break;  // uniform: set before the barrier above
       max_pass();
     }
     // (m, l) with l in [1, 2): the reference is not the maximum, so l may be far from 1
