@@ -154,10 +154,10 @@ sparse_mqa_latent_kernel(const AttnParams p) {
     // the selection's LDS lies behind the list
     static_assert(SKPT * NT == 8192, "the selecting instance takes up to 8192 scores");
     int* const h1 = reinterpret_cast<int*>(smem + 4 * 8 * NT);
-    int* const h2 = h1 + kBins * kSub1;
+    int* const h2 = h1 + kHist1<NT>;
     int* const h3 = h2 + kBins;
     int* const sw = h3 + kBins / 2;
-    static_assert(4 * 8 * NT + (kBins * kSub1 + kBins + kBins / 2 + 16) * 4 <= M::PB, "selection LDS");
+    static_assert(4 * 8 * NT + (kHist1<NT> + kBins + kBins / 2 + 16) * 4 <= M::PB, "selection LDS");
     const RowSelLds lds{h1, h2, h3, sw, sw + 8, sw + 12};
     const int G = static_cast<int>(p.G), k = p.topk;
     const bool search = G > k;
@@ -177,14 +177,28 @@ sparse_mqa_latent_kernel(const AttnParams p) {
     int need_eq;
     row_sel_threshold<SKPT, NT>(key, search, k, lds, T, need_eq);
     const RowTake tk = row_sel_take<SKPT, NT>(key, T, need_eq, sw);
-    // the list is in the top-k launch's form by construction: planned over its valid entries,
-    // every thread's picks straight to their places (one predicated store per key, no walk over
-    // the picks: a thread may hold 32 of them)
+    // The selection is bound by one wave's chain of instructions per SIMD (32 scores per thread,
+    // some 10 K of a short step's 40 K cycles), so nothing in it is conditional per key: see
+    // the spare words of topk_core.h.  The launch, against conditional counts and stores and
+    // first-level counters side by side: one row over 8192 keys 21.0 -> 19.0 us, 8 rows 24.2 ->
+    // 22.5, 32 rows 38.8 -> 36.8, one row over 512 keys 14.4 -> 13.6.
+    // The list is in the top-k launch's form by construction: planned over its valid entries.
+    // A thread's picks take list positions pos .. pos + popcount - 1, ascending with the
+    // thread, so only the threads around this split's slice walk them -- and every thread of
+    // the row's first workgroup, which writes the list
     rp.plan_split(p, tk.written);
+    const bool lists = p.sel_out != nullptr && rp.split == 0 && rp.hgrp == 0;
+    if (lists || (tk.pos < rp.v_end - rp.nwd && tk.pos + __builtin_popcount(tk.sel) > rp.sp_begin)) {
+      int* const spare = row_sel_spare<NT>(lds, lane);
+      int at = tk.pos;
 #pragma unroll
-    for (int j = 0; j < SKPT; ++j)
-      if ((tk.sel >> j) & 1u) sidx[tk.pos + __builtin_popcount(tk.sel & ((1u << j) - 1u))] = i0 + j;
-    if (p.sel_out != nullptr && rp.split == 0 && rp.hgrp == 0) {  // the row's first workgroup writes the list
+      for (int j = 0; j < SKPT; ++j) {
+        const int take = static_cast<int>((tk.sel >> j) & 1u);
+        *(take ? sidx + at : spare) = i0 + j;
+        at += take;
+      }
+    }
+    if (lists) {
       lds_barrier();
       int32_t* const orow = p.sel_out + rp.row * p.sel_out_stride;
       for (int i = 4 * tid; i < k; i += 4 * NT) {

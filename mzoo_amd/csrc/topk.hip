@@ -213,7 +213,7 @@ __global__ void __launch_bounds__(NT) topk_row_kernel(const float* __restrict__ 
                                                       int k, int32_t* __restrict__ out, int64_t out_stride,
                                                       SlotMap sm = SlotMap{}) {
   constexpr int NW = NT / 64;
-  __shared__ __align__(16) int hist1[kBins * kSub1];
+  __shared__ __align__(16) int hist1[kHist1<NT>];
   __shared__ __align__(16) int hist2[kBins];
   __shared__ __align__(16) int hist3[kBins / 2];
   __shared__ int wsum[NW];

@@ -94,21 +94,39 @@ __device__ __forceinline__ BinHit find_bin(const int (&c)[NB / NT], int rem, int
   for (int j = 0; j < BPT; ++j) s += c[j];
   int total;
   const int incl = block_incl_scan<NT>(s, wsum, total);
-  int above = incl - s;
+  const int above = incl - s;
+  if (above < rem && rem <= incl) {  // exactly one thread when rem <= total
+    // the first of its bins whose inclusive count reaches rem (no branch per bin)
+    int past = 0, before = above, upto = above, run = above;
 #pragma unroll
-  for (int j = 0; j < BPT; ++j) {
-    if (above < rem && rem <= above + c[j]) {  // exactly one (thread, j) when rem <= total
-      sh[0] = NB - 1 - (BPT * tid + j);
-      sh[1] = rem - above;
-      sh[2] = c[j];
+    for (int j = 0; j < BPT; ++j) {
+      const bool open = run < rem;  // no bin before j reached rem
+      before = open ? run : before;
+      run += c[j];
+      upto = open ? run : upto;
+      past += run < rem ? 1 : 0;
     }
-    above += c[j];
+    sh[0] = NB - 1 - (BPT * tid + past);
+    sh[1] = rem - before;
+    sh[2] = upto - before;
   }
   lds_barrier();
   return BinHit{sh[0], sh[1], sh[2], total};
 }
 
-// The LDS of one row's selection: hist1 [kBins * kSub1], hist2 [kBins] (bits 20..10 of the
+// The first level's counters: from 512 threads a bin's kSub1 sub-counters side by side, which a
+// thread reads as one int4 a bin.  With 256 threads a thread owns 8 bins, whose int4s would
+// lie 128 bytes from the next thread's (8 lanes to a bank), so there each sub-counter has a plane
+// of its own, 16 banks on from the last: two int4s a plane, two lanes to a bank.  The 4 x 16
+// counters between the planes are one spare word per lane (row_sel_spare), where a lane counts
+// a key that is not to be counted: with one wave per SIMD a conditional store costs the
+// round trip through the execution mask, some 70 cycles a key.
+template <int NT>
+constexpr int kHist1Plane = NT >= 512 ? 1 : kBins + 16;
+template <int NT>
+constexpr int kHist1 = NT >= 512 ? kBins * kSub1 : kHist1Plane<NT> * kSub1;
+
+// The LDS of one row's selection: hist1 [kHist1<NT>], hist2 [kBins] (bits 20..10 of the
 // keys in the first level's bin), hist3 [kBins / 2] (bits 9..0 of the keys in the second
 // level's bin), all 16-byte aligned; wsum [NT / 64]; sh0, sh1 [3] each (the bin searches
 // alternate between the two).
@@ -120,9 +138,39 @@ struct RowSelLds {
   int* sh0;
   int* sh1;
 };
+
+// Thread t's counts of bins NB-1-(BPT*t+j), summed over `planes` copies of the histogram
+// `stride` counters apart.  A thread's bins are contiguous: read in whole int4s where there are
+// that many.
+template <int NT, int NB, int PLANES = 1>
+__device__ __forceinline__ void bin_counts(const int* hist, int stride, int tid, int (&c)[NB / NT]) {
+  constexpr int BPT = NB / NT;
+  const int* at = hist + (NB - BPT * (tid + 1));
+#pragma unroll
+  for (int j = 0; j < BPT; ++j) c[j] = 0;
+#pragma unroll
+  for (int q = 0; q < PLANES; ++q) {
+    if constexpr (BPT % 4 == 0) {
+#pragma unroll
+      for (int j = 0; j < BPT; j += 4) {
+        const int4 v = *reinterpret_cast<const int4*>(at + q * stride + j);
+        c[BPT - 1 - j] += v.x;
+        c[BPT - 2 - j] += v.y;
+        c[BPT - 3 - j] += v.z;
+        c[BPT - 4 - j] += v.w;
+      }
+    } else {
+#pragma unroll
+      for (int j = 0; j < BPT; ++j) c[BPT - 1 - j] += at[q * stride + j];
+    }
+  }
+}
+
+// A lane's spare word (256 threads; not cleared, not read).
 template <int NT>
-constexpr int row_sel_lds_bytes() {
-  return (kBins * kSub1 + kBins + kBins / 2 + NT / 64 + 8) * 4;
+__device__ __forceinline__ int* row_sel_spare(const RowSelLds& s, int lane) {
+  static_assert(kHist1Plane<NT> > 1, "the spare words lie between the planes");
+  return s.hist1 + (lane & (kSub1 - 1)) * kHist1Plane<NT> + kBins + lane / kSub1;
 }
 
 // Clear the three histograms (no barrier: the caller's next barrier publishes it; issue it
@@ -130,7 +178,7 @@ constexpr int row_sel_lds_bytes() {
 template <int NT>
 __device__ __forceinline__ void row_sel_clear(const RowSelLds& s, int tid) {
   int4* h4 = reinterpret_cast<int4*>(s.hist1);
-  for (int i = tid; i < kBins * kSub1 / 4; i += NT) h4[i] = int4{0, 0, 0, 0};
+  for (int i = tid; i < kHist1<NT> / 4; i += NT) h4[i] = int4{0, 0, 0, 0};
   for (int i = tid; i < kBins / 4; i += NT) reinterpret_cast<int4*>(s.hist2)[i] = int4{0, 0, 0, 0};
   for (int i = tid; i < kBins / 8; i += NT) reinterpret_cast<int4*>(s.hist3)[i] = int4{0, 0, 0, 0};
 }
@@ -142,26 +190,33 @@ template <int KPT, int NT>
 __device__ __forceinline__ void row_sel_threshold(const uint32_t (&key)[KPT], bool search, int k, const RowSelLds& s,
                                                   uint32_t& T, int& need_eq) {
   constexpr int BPT = kBins / NT;
+  constexpr bool kPlanes = kHist1Plane<NT> > 1;
   const int tid = threadIdx.x;
   const int lane = tid & 63;
   BinHit h1{0, 0, 0, 0};
   if (search) {
-    int* hl = s.hist1 + (lane & (kSub1 - 1));
+    int* hl = s.hist1 + (lane & (kSub1 - 1)) * kHist1Plane<NT>;
 #pragma unroll
-    for (int j = 0; j < KPT; ++j)
-      if (key[j] > kNegInfKey) atomicAdd(hl + (key[j] >> kLowBits) * kSub1, 1);
+    for (int j = 0; j < KPT; ++j) {
+      if constexpr (kPlanes) atomicAdd(key[j] > kNegInfKey ? hl + (key[j] >> kLowBits) : row_sel_spare<NT>(s, lane), 1);
+      else if (key[j] > kNegInfKey) atomicAdd(hl + (key[j] >> kLowBits) * kSub1, 1);
+    }
     lds_barrier();
     int c1[BPT];
+    if constexpr (kPlanes) {
+      bin_counts<NT, kBins, kSub1>(s.hist1, kHist1Plane<NT>, tid, c1);
+    } else {
 #pragma unroll
-    for (int j = 0; j < BPT; ++j) {
-      const int4* hb = reinterpret_cast<const int4*>(s.hist1) + (kBins - 1 - (BPT * tid + j)) * (kSub1 / 4);
-      int sum = 0;
+      for (int j = 0; j < BPT; ++j) {
+        const int4* hb = reinterpret_cast<const int4*>(s.hist1) + (kBins - 1 - (BPT * tid + j)) * (kSub1 / 4);
+        int sum = 0;
 #pragma unroll
-      for (int q = 0; q < kSub1 / 4; ++q) {
-        const int4 v = hb[q];
-        sum += (v.x + v.y) + (v.z + v.w);
+        for (int q = 0; q < kSub1 / 4; ++q) {
+          const int4 v = hb[q];
+          sum += (v.x + v.y) + (v.z + v.w);
+        }
+        c1[j] = sum;
       }
-      c1[j] = sum;
     }
     h1 = find_bin<NT, kBins>(c1, k, s.wsum, s.sh0);
   }
@@ -173,12 +228,14 @@ __device__ __forceinline__ void row_sel_threshold(const uint32_t (&key)[KPT], bo
       T = (b1 << kLowBits) - 1u;
     } else {
 #pragma unroll
-      for (int j = 0; j < KPT; ++j)
-        if ((key[j] >> kLowBits) == b1) atomicAdd(&s.hist2[(key[j] >> 10) & (kBins - 1)], 1);
+      for (int j = 0; j < KPT; ++j) {
+        int* const at = s.hist2 + ((key[j] >> 10) & (kBins - 1));
+        if constexpr (kPlanes) atomicAdd((key[j] >> kLowBits) == b1 ? at : row_sel_spare<NT>(s, lane), 1);
+        else if ((key[j] >> kLowBits) == b1) atomicAdd(at, 1);
+      }
       lds_barrier();
       int c2[BPT];
-#pragma unroll
-      for (int j = 0; j < BPT; ++j) c2[j] = s.hist2[kBins - 1 - (BPT * tid + j)];
+      bin_counts<NT, kBins>(s.hist2, 0, tid, c2);
       const BinHit h2 = find_bin<NT, kBins>(c2, h1.rem, s.wsum, s.sh1);
       const uint32_t p2 = (b1 << kLowBits) | (static_cast<uint32_t>(h2.bin) << 10);
       if (h2.count == h2.rem) {
@@ -190,8 +247,7 @@ __device__ __forceinline__ void row_sel_threshold(const uint32_t (&key)[KPT], bo
         lds_barrier();
         constexpr int B3 = kBins / 2;
         int c3[B3 / NT];
-#pragma unroll
-        for (int j = 0; j < B3 / NT; ++j) c3[j] = s.hist3[B3 - 1 - ((B3 / NT) * tid + j)];
+        bin_counts<NT, B3>(s.hist3, 0, tid, c3);
         const BinHit h3 = find_bin<NT, B3>(c3, h2.rem, s.wsum, s.sh0);
         T = p2 | static_cast<uint32_t>(h3.bin);  // the k-th largest key itself
         need_eq = h3.rem;
@@ -213,9 +269,13 @@ __device__ __forceinline__ RowTake row_sel_take(const uint32_t (&key)[KPT], uint
   static_assert(KPT * NT <= 32768, "packed counts: at most 2^15 keys per row");
   uint32_t gt_mask = 0u, eq_mask = 0u;
 #pragma unroll
-  for (int j = 0; j < KPT; ++j) {
-    gt_mask |= static_cast<uint32_t>(key[j] > T) << j;
-    eq_mask |= static_cast<uint32_t>((key[j] == T) && (T != kNegInfKey)) << j;
+  for (int j = 0; j < KPT; ++j) gt_mask |= static_cast<uint32_t>(key[j] > T) << j;
+  // need_eq != 0 (workgroup-uniform) only where T is a key.  Several waves per SIMD compare all the
+  // same: a branch here cost rows of 32 keys x 1024 threads 13.5 -> 14.8 us, and gained
+  // rows of 8 keys x 256 threads 5.1 -> 4.9
+  if (NT > 256 || need_eq != 0) {
+#pragma unroll
+    for (int j = 0; j < KPT; ++j) eq_mask |= static_cast<uint32_t>((key[j] == T) && (T != kNegInfKey)) << j;
   }
   const int n_gt = __builtin_popcount(gt_mask), n_eq = __builtin_popcount(eq_mask);
   // packed as unsigned: n_gt <= G <= 32768 fills bit 31 at most, n_eq stays below 2^16

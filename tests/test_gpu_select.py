@@ -146,3 +146,36 @@ def test_select_graph_replays(dev):
         ref_o, ref_l, ref_i = _two_launches(qd, pos_d, win_c, main_c, None, scd, topk, skd, nsplit, rope)
         torch.cuda.synchronize()
         assert torch.equal(idx, ref_i) and torch.equal(out, ref_o) and torch.equal(lse, ref_l), f"replay {rep}"
+
+
+def _spread(kind, b, g, gen):
+    """Scores whose k-th largest key is found at the first, second or third level of bins, or
+    only among equal keys."""
+    base = torch.full((b, g), 0x3F800000, dtype=torch.int32)  # 1.0
+    if kind == "octaves":          # every key in a first-level bin of its own sort
+        return torch.randn(b, g, generator=gen) * torch.exp2(torch.randint(-60, 60, (b, g), generator=gen).float())
+    if kind == "one bin":          # equal in the top 11 bits
+        return (base + torch.randint(0, 1 << 21, (b, g), generator=gen, dtype=torch.int32)).view(torch.float32)
+    if kind == "low bits":         # equal in all but the last 10 bits: many equal keys too
+        return (base + torch.randint(0, 1 << 10, (b, g), generator=gen, dtype=torch.int32)).view(torch.float32)
+    if kind == "few":              # four values
+        return torch.tensor([-1.0, 0.0, 0.5, 1.0])[torch.randint(0, 4, (b, g), generator=gen)]
+    return torch.full((b, g), 0.25)  # "equal"
+
+
+@pytest.mark.parametrize("kind", ["octaves", "one bin", "low bits", "few", "equal"])
+@pytest.mark.parametrize("g,topk", [(4, 4), (260, 128), (2048, 512), (2052, 512), (8192, 2048), (8192, 4), (8188, 1000)])
+def test_selected_list_at_every_level(dev, kind, g, topk):
+    """The selection of 256 threads (the attention's own, and the top-k launch up to 2048 keys)
+    against the oracle, with -inf entries between."""
+    b = 2
+    gen = torch.Generator().manual_seed(g + topk)
+    q, win_c, main_c, _, _, sinks = _case(dev, b, g, 4 * g + 3, seed=g)
+    sc = _spread(kind, b, g, gen)
+    sc[1, torch.rand(g, generator=gen) < 0.4] = float("-inf")
+    want = OA.topk_indices(sc.numpy()[:, None], topk)[:, 0]
+    pos_d = torch.full((b,), 4 * g + 3, dtype=torch.int64, device=dev)
+    _, _, idx = MA.sparse_mqa_decode_select(q.to(dev), pos_d, win_c, 128, main_cache=main_c, scores=sc.to(dev),
+                                            topk=topk, sinks=sinks.to(dev), nsplit=3)
+    assert np.array_equal(idx.cpu().numpy(), want)
+    assert np.array_equal(MI.topk(sc.to(dev), topk).cpu().numpy(), want)
