@@ -122,14 +122,17 @@ __global__ void __launch_bounds__(256) compress_kernel(const float* __restrict__
 // 889 -> 62.8 us, at ratio 8 59 -> 14.5, at ratio 3 30 -> 24 (16 tokens ahead: 59.5, 23.6 and
 // 41.5 us; 4: 72, 16.1 and 19.4).
 constexpr int kTokensAhead = 8;
+constexpr int64_t kWideGridX = int64_t(1) << 21;  // groups along the grid's x
 
 template <int ODT, int WDT>
 __global__ void __launch_bounds__(64 * kMaxPerLane)
-    compress_wide_kernel(const float* __restrict__ kv, const float* __restrict__ gate, int64_t n_groups, int ratio, int D,
-                         int64_t tokens_per_batch, const void* __restrict__ weight, float eps, void* __restrict__ out) {
+    compress_wide_kernel(const float* __restrict__ kv, const float* __restrict__ gate, int64_t groups, int64_t n_groups,
+                         int ratio, int D, int64_t tokens_per_batch, const void* __restrict__ weight, float eps,
+                         void* __restrict__ out) {
   __shared__ float h_lds[64 * kMaxPerLane];
   __shared__ float inv_lds;
-  const int64_t rid = blockIdx.x;
+  const int64_t rid = static_cast<int64_t>(blockIdx.y) * gridDim.x + blockIdx.x;
+  if (rid >= groups) return;
   const int64_t b = rid / n_groups;
   const int64_t g = rid - b * n_groups;
   const int d = threadIdx.x < D ? threadIdx.x : D - 1;  // (threads beyond D: a channel again, dropped)
@@ -266,9 +269,12 @@ void launch_compress_r(const float* kv, const float* gate, int64_t B, int64_t n,
     case 1: compress_kernel<ODT, WDT, 1><<<grid, 256, 0, s>>>(kv, gate, B, n, ratio, D, tpb, w, eps, out); break;
     case 2: compress_kernel<ODT, WDT, 2><<<grid, 256, 0, s>>>(kv, gate, B, n, ratio, D, tpb, w, eps, out); break;
     case 4: compress_kernel<ODT, WDT, 4><<<grid, 256, 0, s>>>(kv, gate, B, n, ratio, D, tpb, w, eps, out); break;
-    default:
-      compress_wide_kernel<ODT, WDT><<<static_cast<unsigned>(B * n), (D + 63) / 64 * 64, 0, s>>>(kv, gate, n, ratio, D, tpb,
-                                                                                               w, eps, out);
+    default: {
+      // a launch takes fewer than 2^32 threads along x (4 M groups of 1024): the rest along y
+      const int64_t groups = B * n, x = groups < kWideGridX ? groups : kWideGridX;
+      const dim3 wide(static_cast<unsigned>(x), static_cast<unsigned>((groups + x - 1) / x));
+      compress_wide_kernel<ODT, WDT><<<wide, (D + 63) / 64 * 64, 0, s>>>(kv, gate, groups, n, ratio, D, tpb, w, eps, out);
+    }
   }
 }
 

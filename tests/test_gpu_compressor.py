@@ -88,3 +88,22 @@ def test_rope_bit_exact(dev, dtype):
                                       inverse=inverse)
         want = C.rope(x.float().numpy(), cos[:, :, None], sin[:, :, None], inverse, NAMES[dtype])
         assert np.array_equal(_bits(got), _obits(want, dtype))
+
+
+def test_compress_more_threads_than_one_grid_axis(dev):
+    """From 2^32 threads (here 34 M groups of 65 channels, 128 threads each) the launch takes a
+    second grid axis: the groups at both ends and around its turns equal those of small calls.
+    One tensor of 26 GB is the projection and the gate, zero but in those groups."""
+    d, ratio, n = 65, 3, (1 << 25) + 5
+    if torch.cuda.mem_get_info(dev)[0] < (40 << 30):
+        pytest.skip("needs 40 GB of GPU memory")
+    gen = torch.Generator().manual_seed(3)
+    starts = [0, (1 << 21) - 2, (1 << 22) - 2, (1 << 24) - 2, (1 << 25) - 2, n - 2]
+    kv = torch.zeros(1, n * ratio, d, device=dev)
+    w = (1 + 0.1 * torch.randn(d, generator=gen)).bfloat16().to(dev)
+    for g in starts:
+        kv[:, g * ratio:(g + 4) * ratio].copy_(torch.randn(1, min(4, n - g) * ratio, d, generator=gen).to(dev))
+    out = MC.compress(kv, kv, ratio, w, 1e-6, torch.bfloat16)
+    for g in starts:
+        part = kv[:, g * ratio:(g + 4) * ratio]
+        assert torch.equal(out[:, g:g + 4], MC.compress(part, part, ratio, w, 1e-6, torch.bfloat16)), f"groups {g}.."
