@@ -26,6 +26,15 @@ namespace {
 constexpr int kMaxPerLane = 16;  // D <= 1024
 constexpr int kPoolAhead = 2;    // channels per lane loaded together (2 * ratio registers each)
 
+// Blocks along the grid's x, which takes fewer than 2^32 threads (2^21 blocks of 1024); the rest
+// along y.
+constexpr int64_t kGridX = int64_t(1) << 21;
+inline dim3 grid_xy(int64_t blocks) {
+  const int64_t x = blocks < kGridX ? blocks : kGridX;
+  return dim3(static_cast<unsigned>(x), static_cast<unsigned>((blocks + x - 1) / x));
+}
+__device__ __forceinline__ int64_t block_xy() { return static_cast<int64_t>(blockIdx.y) * gridDim.x + blockIdx.x; }
+
 // The pooled value of one channel over R tokens held in registers: the operations and order
 // above; exp(g_r - max) is formed once and used in the sum and in the weight.
 template <int R>
@@ -46,10 +55,11 @@ __device__ __forceinline__ float pool_channel(const float (&k)[R], const float (
   return acc;
 }
 
-// Ratios 1, 2 and 4: one wave per group, kPoolAhead channels' whole groups loaded into
-// registers before the first is used.  It was bound by latency -- loops that read each gate
-// three times from the cache, one load in flight, and formed each exp twice; now by the
-// divisions and exps (some 55 operations per token and channel), about twice its memory time.
+// Ratios 1, 2 and 4, and 3 and 5 from wave_groups() groups: one wave per group, kPoolAhead
+// channels' whole groups loaded into registers before the first is used.  It was bound by
+// latency -- loops that read each gate three times from the cache, one load in flight, and
+// formed each exp twice; now by the divisions and exps (some 55 operations per token and
+// channel), about twice its memory time.
 // 8192 tokens x 576 channels: ratio 4 35.9 -> 14.0 us, ratio 2 24.3 -> 13.6 us (4 channels
 // ahead 14.2, 8 15.3, 16 15.4).
 template <int ODT, int WDT, int RATIO>
@@ -58,7 +68,7 @@ __global__ void __launch_bounds__(256) compress_kernel(const float* __restrict__
                                                        int64_t tokens_per_batch, const void* __restrict__ weight,
                                                        float eps, void* __restrict__ out) {
   const int lane = threadIdx.x & 63;
-  const int64_t rid = static_cast<int64_t>(blockIdx.x) * 4 + (threadIdx.x >> 6);
+  const int64_t rid = block_xy() * 4 + (threadIdx.x >> 6);
   if (rid >= B * n_groups) return;  // whole waves
   const int64_t b = rid / n_groups;
   const int64_t g = rid - b * n_groups;
@@ -115,14 +125,20 @@ __global__ void __launch_bounds__(256) compress_kernel(const float* __restrict__
   }
 }
 
-// Any other ratio: one workgroup per group, thread d owns channel d and walks the group's
-// tokens in order, kTokensAhead of them loaded together; the channels meet in LDS, where wave
-// 0 sums their squares in the pinned order.  A group of 128 tokens in one wave took 9 channels
-// x 128 tokens x 3 dependent reads per lane in turn: 8192 tokens x 576 channels at ratio 128
-// 889 -> 62.8 us, at ratio 8 59 -> 14.5, at ratio 3 30 -> 24 (16 tokens ahead: 59.5, 23.6 and
-// 41.5 us; 4: 72, 16.1 and 19.4).
+// Any other ratio, and ratios 3 and 5 of fewer groups: one workgroup per group, thread d owns
+// channel d and walks the group's tokens in order, kTokensAhead of them loaded together; the
+// channels meet in LDS, where wave 0 sums their squares in the pinned order.  A group of 128
+// tokens in one wave took 9 channels x 128 tokens x 3 dependent reads per lane in turn: 8192
+// tokens x 576 channels at ratio 128 889 -> 62.8 us, at ratio 8 59 -> 14.5 (16 tokens ahead:
+// 59.5 and 23.6 us; 4: 72 and 16.1).
 constexpr int kTokensAhead = 8;
-constexpr int64_t kWideGridX = int64_t(1) << 21;  // groups along the grid's x
+
+// Ratios 3 and 5 in the wave form: from here, a wave or more for each SIMD, it keeps the chip
+// busy, and it reads a short group's tokens once, where the workgroup form requests 8 at a time
+// three times over.  Workgroup -> wave form, us: ratio 3, 576 channels, 1000 groups 9.2 -> 8.6 (682:
+// 7.5 -> 8.6), 2730 24.1 -> 13.4, 21845 188 -> 68; 1024 channels, 1000 groups 13.4 -> 13.1 (682: 10.8 ->
+// 12.7); ratio 5, 1024 channels, 1638 groups 26.7 -> 23.5 (1200: 20.3 -> 22.7), 13107 197 -> 123.
+constexpr int64_t wave_groups(int ratio) { return 256 * (ratio + 1); }
 
 template <int ODT, int WDT>
 __global__ void __launch_bounds__(64 * kMaxPerLane)
@@ -131,7 +147,7 @@ __global__ void __launch_bounds__(64 * kMaxPerLane)
                          void* __restrict__ out) {
   __shared__ float h_lds[64 * kMaxPerLane];
   __shared__ float inv_lds;
-  const int64_t rid = static_cast<int64_t>(blockIdx.y) * gridDim.x + blockIdx.x;
+  const int64_t rid = block_xy();
   if (rid >= groups) return;
   const int64_t b = rid / n_groups;
   const int64_t g = rid - b * n_groups;
@@ -264,17 +280,17 @@ __global__ void rope_kernel(const void* __restrict__ x, const float* __restrict_
 template <int ODT, int WDT>
 void launch_compress_r(const float* kv, const float* gate, int64_t B, int64_t n, int ratio, int D, int64_t tpb,
                        const void* w, float eps, void* out, hipStream_t s) {
-  const unsigned grid = static_cast<unsigned>((B * n + 3) / 4);
-  switch (ratio) {
+  const dim3 grid = grid_xy((B * n + 3) / 4);
+  const bool wide = (ratio == 3 || ratio == 5) && B * n < wave_groups(ratio);
+  switch (wide ? 0 : ratio) {
     case 1: compress_kernel<ODT, WDT, 1><<<grid, 256, 0, s>>>(kv, gate, B, n, ratio, D, tpb, w, eps, out); break;
     case 2: compress_kernel<ODT, WDT, 2><<<grid, 256, 0, s>>>(kv, gate, B, n, ratio, D, tpb, w, eps, out); break;
+    case 3: compress_kernel<ODT, WDT, 3><<<grid, 256, 0, s>>>(kv, gate, B, n, ratio, D, tpb, w, eps, out); break;
     case 4: compress_kernel<ODT, WDT, 4><<<grid, 256, 0, s>>>(kv, gate, B, n, ratio, D, tpb, w, eps, out); break;
-    default: {
-      // a launch takes fewer than 2^32 threads along x (4 M groups of 1024): the rest along y
-      const int64_t groups = B * n, x = groups < kWideGridX ? groups : kWideGridX;
-      const dim3 wide(static_cast<unsigned>(x), static_cast<unsigned>((groups + x - 1) / x));
-      compress_wide_kernel<ODT, WDT><<<wide, (D + 63) / 64 * 64, 0, s>>>(kv, gate, groups, n, ratio, D, tpb, w, eps, out);
-    }
+    case 5: compress_kernel<ODT, WDT, 5><<<grid, 256, 0, s>>>(kv, gate, B, n, ratio, D, tpb, w, eps, out); break;
+    default:
+      compress_wide_kernel<ODT, WDT><<<grid_xy(B * n), (D + 63) / 64 * 64, 0, s>>>(kv, gate, B * n, n, ratio, D, tpb, w, eps,
+                                                                                   out);
   }
 }
 

@@ -90,13 +90,25 @@ def test_rope_bit_exact(dev, dtype):
         assert np.array_equal(_bits(got), _obits(want, dtype))
 
 
+@pytest.mark.parametrize("ratio,groups,d", [(3, 1023, 100), (3, 1024, 65), (3, 1025, 1), (5, 1535, 64), (5, 1539, 576),
+                                            (3, 1024, 1024)])
+def test_compress_forms_of_ratios_3_and_5(dev, ratio, groups, d):
+    """On both sides of the line between the workgroup and the wave form: the oracle's bits."""
+    gen = torch.Generator().manual_seed(groups + d)
+    kv, gate = torch.randn(1, groups * ratio, d, generator=gen), torch.randn(1, groups * ratio, d, generator=gen) * 5
+    w = (1 + 0.1 * torch.randn(d, generator=gen)).bfloat16()
+    got = MC.compress(kv.to(dev), gate.to(dev), ratio, w.to(dev), 1e-6, torch.bfloat16)
+    want = C.compress(kv.numpy(), gate.numpy(), ratio, w.float().numpy(), 1e-6, "bfloat16")
+    assert np.array_equal(_bits(got), _obits(want, torch.bfloat16))
+
+
 def test_compress_more_threads_than_one_grid_axis(dev):
     """From 2^32 threads (here 34 M groups of 65 channels, 128 threads each) the launch takes a
     second grid axis: the groups at both ends and around its turns equal those of small calls.
-    One tensor of 26 GB is the projection and the gate, zero but in those groups."""
-    d, ratio, n = 65, 3, (1 << 25) + 5
-    if torch.cuda.mem_get_info(dev)[0] < (40 << 30):
-        pytest.skip("needs 40 GB of GPU memory")
+    One tensor of 52 GB is the projection and the gate, zero but in those groups."""
+    d, ratio, n = 65, 6, (1 << 25) + 5
+    if torch.cuda.mem_get_info(dev)[0] < (64 << 30):
+        pytest.skip("needs 64 GB of GPU memory")
     gen = torch.Generator().manual_seed(3)
     starts = [0, (1 << 21) - 2, (1 << 22) - 2, (1 << 24) - 2, (1 << 25) - 2, n - 2]
     kv = torch.zeros(1, n * ratio, d, device=dev)
