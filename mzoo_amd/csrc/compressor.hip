@@ -155,27 +155,27 @@ __global__ void __launch_bounds__(64 * kMaxPerLane)
   const float* k = kv + (b * tokens_per_batch + g * ratio) * D + d;
   const float* gt = gate + (b * tokens_per_batch + g * ratio) * D + d;
   // the group's next tokens (at or beyond its end the last one, not used)
-  auto ahead = [&](const float* p, int r0, float (&v)[kTokensAhead]) __attribute__((always_inline)) {
+  auto ahead = [&](const float* p, int64_t r0, float (&v)[kTokensAhead]) __attribute__((always_inline)) {
 #pragma unroll
-    for (int j = 0; j < kTokensAhead; ++j) v[j] = p[static_cast<int64_t>(r0 + j < ratio ? r0 + j : ratio - 1) * D];
+    for (int j = 0; j < kTokensAhead; ++j) v[j] = p[(r0 + j < ratio ? r0 + j : ratio - 1) * D];
   };
   float gv[kTokensAhead], kvv[kTokensAhead];
   float m = gt[0];
-  for (int r0 = 0; r0 < ratio; r0 += kTokensAhead) {
+  for (int64_t r0 = 0; r0 < ratio; r0 += kTokensAhead) {
     ahead(gt, r0, gv);
 #pragma unroll
     for (int j = 0; j < kTokensAhead; ++j)
       if (r0 + j > 0 && r0 + j < ratio) m = fmaxf(m, gv[j]);
   }
   float s = 0.0f;
-  for (int r0 = 0; r0 < ratio; r0 += kTokensAhead) {
+  for (int64_t r0 = 0; r0 < ratio; r0 += kTokensAhead) {
     ahead(gt, r0, gv);
 #pragma unroll
     for (int j = 0; j < kTokensAhead; ++j)
       if (r0 + j < ratio) s = s + exp_pinned(gv[j] - m);
   }
   float acc = 0.0f;
-  for (int r0 = 0; r0 < ratio; r0 += kTokensAhead) {
+  for (int64_t r0 = 0; r0 < ratio; r0 += kTokensAhead) {
     ahead(gt, r0, gv);
     ahead(k, r0, kvv);
 #pragma unroll
