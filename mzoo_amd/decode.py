@@ -280,9 +280,10 @@ class SparseDecodeLayer:
         fp8 = self.cfg.index_format == "fp8"
         codes, scales = (self.k_codes, self.k_scales.unsqueeze(-1)) if fp8 else (self.k_packed, self.k_e8m0)
         dst = codes[:, start:start + n], scales[:, start:start + n]
-        # one row's groups are contiguous in the cache: quantized straight into it
-        direct = (dst[0].is_contiguous() and dst[1].is_contiguous() and dst[0].shape[:2] == index_keys.shape[:2]
-                  and index_keys.shape[2:] == (self.cfg.index_dim,))
+        # one row's groups are contiguous in the cache: quantized straight into it (keys of another
+        # device are quantized there and copied)
+        direct = (index_keys.device == dst[0].device and dst[0].is_contiguous() and dst[1].is_contiguous()
+                  and dst[0].shape[:2] == index_keys.shape[:2] and index_keys.shape[2:] == (self.cfg.index_dim,))
         out = dst if direct else None
         got = quant.quant_fp8_block(index_keys, self.cfg.index_dim, out=out) if fp8 else quant.quant_mxfp4(index_keys, out=out)
         if not direct:
