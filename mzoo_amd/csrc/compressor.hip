@@ -154,33 +154,40 @@ __global__ void __launch_bounds__(64 * kMaxPerLane)
   const int d = threadIdx.x < D ? threadIdx.x : D - 1;  // (threads beyond D: a channel again, dropped)
   const float* k = kv + (b * tokens_per_batch + g * ratio) * D + d;
   const float* gt = gate + (b * tokens_per_batch + g * ratio) * D + d;
-  // the group's next tokens (at or beyond its end the last one, not used)
-  auto ahead = [&](const float* p, int64_t r0, float (&v)[kTokensAhead]) __attribute__((always_inline)) {
+  // kTokensAhead tokens from p on, of which `left` are the group's (beyond them its last, not
+  // used).  The walks count the tokens left and move the pointer: the count cannot wrap at any
+  // ratio, and the addresses stay 32-bit offsets (a 64-bit token number took 8192 tokens of 576 channels
+  // at ratio 128 from 62.8 to 70.7 us, at ratio 8 from 15.4 to 16.6; so counted 63.4 and 15.8).
+  const int step = kTokensAhead * D;
+  auto ahead = [&](const float* p, int left, float (&v)[kTokensAhead]) __attribute__((always_inline)) {
 #pragma unroll
-    for (int j = 0; j < kTokensAhead; ++j) v[j] = p[(r0 + j < ratio ? r0 + j : ratio - 1) * D];
+    for (int j = 0; j < kTokensAhead; ++j) v[j] = p[(j < left ? j : left - 1) * D];
   };
   float gv[kTokensAhead], kvv[kTokensAhead];
+  const float* at = gt;
   float m = gt[0];
-  for (int64_t r0 = 0; r0 < ratio; r0 += kTokensAhead) {
-    ahead(gt, r0, gv);
+  for (int left = ratio; left > 0; left -= kTokensAhead, at += step) {
+    ahead(at, left, gv);
 #pragma unroll
     for (int j = 0; j < kTokensAhead; ++j)
-      if (r0 + j > 0 && r0 + j < ratio) m = fmaxf(m, gv[j]);
+      if (j < left) m = fmaxf(m, gv[j]);
   }
+  at = gt;
   float s = 0.0f;
-  for (int64_t r0 = 0; r0 < ratio; r0 += kTokensAhead) {
-    ahead(gt, r0, gv);
+  for (int left = ratio; left > 0; left -= kTokensAhead, at += step) {
+    ahead(at, left, gv);
 #pragma unroll
     for (int j = 0; j < kTokensAhead; ++j)
-      if (r0 + j < ratio) s = s + exp_pinned(gv[j] - m);
+      if (j < left) s = s + exp_pinned(gv[j] - m);
   }
+  at = gt;
   float acc = 0.0f;
-  for (int64_t r0 = 0; r0 < ratio; r0 += kTokensAhead) {
-    ahead(gt, r0, gv);
-    ahead(k, r0, kvv);
+  for (int left = ratio; left > 0; left -= kTokensAhead, at += step, k += step) {
+    ahead(at, left, gv);
+    ahead(k, left, kvv);
 #pragma unroll
     for (int j = 0; j < kTokensAhead; ++j)
-      if (r0 + j < ratio) acc = acc + kvv[j] * div_rn(exp_pinned(gv[j] - m), s);
+      if (j < left) acc = acc + kvv[j] * div_rn(exp_pinned(gv[j] - m), s);
   }
   const float v = round_to_dtype<ODT>(acc);  // latent.to(dtype) before the norm
   h_lds[threadIdx.x] = v;
