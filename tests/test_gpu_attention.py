@@ -185,22 +185,28 @@ def test_decode_fp8_config2_shape(dev, nsplit):
     torch.testing.assert_close(lse.cpu(), ref_lse, **LSE_TOL)
 
 
-def test_decode_table_kernels_agree_bitwise(dev):
-    """A launch whose longest possible split keeps every entry table runs the kernel instance
-    without the table ring; the same rows through the ring-capable instance -- a longer index
-    list (top-k form: ascending picks, then -1) with the same valid prefix, so its workgroups
-    build all their tables at run time -- give the same bits, and both match the oracle."""
+def test_decode_list_paths_agree_bitwise(dev):
+    """The entry table from a list requested ahead (at most 2048 entries, a multiple of 4, rows
+    16-byte aligned; trimmed to its valid prefix) and from a list read from memory as the table
+    is built (longer, of another length, or unaligned; its trailing empty slots stay, as masked
+    entries): the same 300 picks give the same bits over one split, and the oracle's result."""
     b, h, gcap, pos = 4, 128, 8192, 32767
     q, win_c, main_c, _, _, sinks, g = _decode_case(dev, b, h, gcap, 2048, pos, seed=41)
     gen = torch.Generator().manual_seed(42)
     picks = torch.stack([torch.randperm(g, generator=gen)[:300].sort().values for _ in range(b)]).int()
-    short = torch.cat([picks, torch.full((b, 20), -1, dtype=torch.int32)], 1)  # 128 + 320 entries at most
-    full = torch.cat([picks, torch.full((b, 2048 - 300), -1, dtype=torch.int32)], 1)  # 128 + 2048
+    lists = {n: torch.cat([picks, torch.full((b, n - 300), -1, dtype=torch.int32)], 1) for n in (320, 318, 2048, 2052)}
+    shifted = torch.full((b * 320 + 1,), -1, dtype=torch.int32, device=dev)
+    shifted[1:] = lists[320].to(dev).flatten()
+    unaligned = shifted[1:].view(b, 320)
+    ahead = [lists[320].to(dev), lists[2048].to(dev)]
+    from_memory = [lists[318].to(dev), lists[2052].to(dev), unaligned]
+    assert all(ix.data_ptr() % 16 == 0 for ix in ahead) and unaligned.data_ptr() % 16 == 4
     positions = torch.full((b,), pos, dtype=torch.int64, device=dev)
     outs = [MA.sparse_mqa_decode(q.to(dev), positions, win_c, 128, main_cache=main_c, groups=g,
-                                 indices=ix.to(dev), sinks=sinks.to(dev), nsplit=1) for ix in (short, full)]
-    assert torch.equal(outs[0][0], outs[1][0]) and torch.equal(outs[0][1], outs[1][1])
-    ref, ref_lse = _decode_oracle(q, win_c, main_c, None, short, sinks, pos, 128, 1, g)
+                                 indices=ix, sinks=sinks.to(dev), nsplit=1) for ix in ahead + from_memory]
+    for o, lse in outs[1:]:
+        assert torch.equal(outs[0][0], o) and torch.equal(outs[0][1], lse)
+    ref, ref_lse = _decode_oracle(q, win_c, main_c, None, lists[320], sinks, pos, 128, 1, g)
     assert_attn_close(outs[0][0], ref)
     torch.testing.assert_close(outs[0][1].cpu(), ref_lse, **LSE_TOL)
 

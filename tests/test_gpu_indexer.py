@@ -201,12 +201,15 @@ def test_fp8_scores_match_oracle(dev, b, s, g, ratio, pos):
 
 
 @pytest.mark.parametrize("b,s,hi,g,ratio,base", [(2, 300, 64, 1000, 4, None), (1, 200, 40, 700, 1, 5000),
-                                                  (1, 128, 64, 64, 4, None), (3, 64, 64, 2048, 4, 0)])
+                                                  (3, 128, 64, 64, 4, None), (3, 64, 64, 2048, 4, 0)])
 def test_fp8_prefill_kernel_matches_row_kernel(dev, b, s, hi, g, ratio, base):
-    """From 64 rows per batch the FP8 scores run the prefill tiling (key tiles held, query
-    rows streamed); it sums in the row kernel's order, so the scores must equal, bit for
-    bit, the row kernel's over chunks of 32 rows with the same positions (ragged row and
-    key counts, fewer than 64 heads, chunked-prefill positions, fully masked key blocks)."""
+    """From 64 rows per batch, and more row workgroups than are resident at once, the FP8
+    scores run the prefill form (query blocks held, keys streamed); it sums in the row kernel's
+    order, so the scores must equal, bit for bit, the row kernel's over chunks of 32 rows with
+    the same positions (ragged row and key counts, fewer than 64 heads, chunked-prefill
+    positions, fully masked key blocks)."""
+    cus = torch.cuda.get_device_properties(dev).multi_processor_count
+    assert b * s * -(-g // 512) > cus * (2 if hi <= 32 else 1), "this case would take the row form"
     q, k, w = _inputs(b, s, hi, 128, g, seed=s + g)
     qc, qs, kc, ks, qd, kd = _fp8_operands(q, k)
     pos = torch.arange(s, dtype=torch.int64).expand(b, s) + (0 if base is None else base)
