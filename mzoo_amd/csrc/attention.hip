@@ -482,12 +482,11 @@ __device__ __forceinline__ void store_o_block(uint16_t* blk, const uint32_t (&w)
   }
 }
 
-// Final bf16 output + lse (one split) or fp32 partials (several) for one lane's head and
-// O^T blocks [b_lo, b_lo + nb): acc[db][j] holds O^T[d][head], d = (b_lo+db)*32 + c_entry(j).
-template <int D, int NOPE, int NDBM>
+// Final bf16 output + lse (one split) or bf16 partials (several) for one lane's head:
+// acc[db][j] holds O^T[d][head], d = db*32 + c_entry(j).
+template <int D, int NOPE, int NB>
 __device__ __forceinline__ void write_result(const AttnParams& p, int64_t row, int64_t b, int split, int head, int half,
-                                             bool lse_lane, int b_lo, int nb, float m_run, float l_run,
-                                             const v16f (&acc)[NDBM]) {
+                                             float m_run, float l_run, const v16f (&acc)[NB]) {
   if (p.write_final) {
     float m_fin = m_run, l_fin = l_run, o_scale;
     if (p.sinks) {
@@ -500,38 +499,35 @@ __device__ __forceinline__ void write_result(const AttnParams& p, int64_t row, i
     } else {
       o_scale = 1.0f / l_fin;
     }
-    uint16_t* orow = p.out + row * p.H * D + static_cast<uint32_t>(head * D + b_lo * 32);
+    uint16_t* orow = p.out + row * p.H * D + static_cast<uint32_t>(head * D);
 #pragma unroll
-    for (int db = 0; db < NDBM; ++db) {
-      if (db < nb) {
-        uint32_t w[8];
+    for (int db = 0; db < NB; ++db) {
+      uint32_t w[8];
 #pragma unroll
-        for (int g4 = 0; g4 < 4; ++g4) {
-          const int d0 = db * 32 + 8 * g4 + 4 * half;
-          uint32_t w0 = f32_to_bf16(acc[db][4 * g4 + 0] * o_scale) |
-                        (static_cast<uint32_t>(f32_to_bf16(acc[db][4 * g4 + 1] * o_scale)) << 16);
-          uint32_t w1 = f32_to_bf16(acc[db][4 * g4 + 2] * o_scale) |
-                        (static_cast<uint32_t>(f32_to_bf16(acc[db][4 * g4 + 3] * o_scale)) << 16);
-          if constexpr (NOPE < D) {
-            // the inverse rotation of the bf16 output (owlet1/attention.py:226)
-            const int ch = b_lo * 32 + d0;
-            if (p.rope_cos && ch >= NOPE) {
-              const int64_t ci = row * ((D - NOPE) / 2) + (ch - NOPE) / 2;
-              const uint32_t cp = *reinterpret_cast<const uint32_t*>(p.rope_cos + ci);
-              const uint32_t sp = *reinterpret_cast<const uint32_t*>(p.rope_sin + ci);
-              w0 = rope_pair_bf16(w0, bf16_to_f32(static_cast<uint16_t>(cp & 0xffffu)),
-                                  -bf16_to_f32(static_cast<uint16_t>(sp & 0xffffu)));
-              w1 = rope_pair_bf16(w1, bf16_to_f32(static_cast<uint16_t>(cp >> 16)),
-                                  -bf16_to_f32(static_cast<uint16_t>(sp >> 16)));
-            }
+      for (int g4 = 0; g4 < 4; ++g4) {
+        const int d0 = db * 32 + 8 * g4 + 4 * half;
+        uint32_t w0 = f32_to_bf16(acc[db][4 * g4 + 0] * o_scale) |
+                      (static_cast<uint32_t>(f32_to_bf16(acc[db][4 * g4 + 1] * o_scale)) << 16);
+        uint32_t w1 = f32_to_bf16(acc[db][4 * g4 + 2] * o_scale) |
+                      (static_cast<uint32_t>(f32_to_bf16(acc[db][4 * g4 + 3] * o_scale)) << 16);
+        if constexpr (NOPE < D) {
+          // the inverse rotation of the bf16 output (owlet1/attention.py:226)
+          if (p.rope_cos && d0 >= NOPE) {
+            const int64_t ci = row * ((D - NOPE) / 2) + (d0 - NOPE) / 2;
+            const uint32_t cp = *reinterpret_cast<const uint32_t*>(p.rope_cos + ci);
+            const uint32_t sp = *reinterpret_cast<const uint32_t*>(p.rope_sin + ci);
+            w0 = rope_pair_bf16(w0, bf16_to_f32(static_cast<uint16_t>(cp & 0xffffu)),
+                                -bf16_to_f32(static_cast<uint16_t>(sp & 0xffffu)));
+            w1 = rope_pair_bf16(w1, bf16_to_f32(static_cast<uint16_t>(cp >> 16)),
+                                -bf16_to_f32(static_cast<uint16_t>(sp >> 16)));
           }
-          w[2 * g4] = w0;
-          w[2 * g4 + 1] = w1;
         }
-        store_o_block(orow + db * 32, w, half);
+        w[2 * g4] = w0;
+        w[2 * g4 + 1] = w1;
       }
+      store_o_block(orow + db * 32, w, half);
     }
-    if (lse_lane) {
+    if (half == 0) {
       const int64_t s_idx = row % p.S;
       p.lse[(b * p.H + head) * p.S + s_idx] = (m_fin + __log2f(l_fin)) * kLn2;
     }
@@ -542,25 +538,23 @@ __device__ __forceinline__ void write_result(const AttnParams& p, int64_t row, i
     const float inv_l = l_run > 0.0f ? 1.0f / l_run : 0.0f;
     uint16_t* pbase = p.part_o + (row * p.split_stride + split) * p.H * static_cast<int64_t>(D);
 #pragma unroll
-    for (int db = 0; db < NDBM; ++db) {
-      if (db < nb) {
-        uint32_t w[8];
+    for (int db = 0; db < NB; ++db) {
+      uint32_t w[8];
 #pragma unroll
-        for (int g4 = 0; g4 < 4; ++g4) {
-          w[2 * g4] = pack_bf16x2(acc[db][4 * g4] * inv_l, acc[db][4 * g4 + 1] * inv_l);
-          w[2 * g4 + 1] = pack_bf16x2(acc[db][4 * g4 + 2] * inv_l, acc[db][4 * g4 + 3] * inv_l);
-        }
-        // groups 2 (b_lo + db) and 2 (b_lo + db) + 1 of the head
-        uint16_t* grp = pbase + static_cast<uint32_t>((b_lo + db) * p.H * 32 + head * 16);
+      for (int g4 = 0; g4 < 4; ++g4) {
+        w[2 * g4] = pack_bf16x2(acc[db][4 * g4] * inv_l, acc[db][4 * g4 + 1] * inv_l);
+        w[2 * g4 + 1] = pack_bf16x2(acc[db][4 * g4 + 2] * inv_l, acc[db][4 * g4 + 3] * inv_l);
+      }
+      // groups 2 db and 2 db + 1 of the head
+      uint16_t* grp = pbase + static_cast<uint32_t>(db * p.H * 32 + head * 16);
 #pragma unroll
-        for (int pr = 0; pr < 2; ++pr) {
-          const auto s0 = __builtin_amdgcn_permlane32_swap(w[4 * pr], w[4 * pr + 2], false, false);
-          const auto s1 = __builtin_amdgcn_permlane32_swap(w[4 * pr + 1], w[4 * pr + 3], false, false);
-          *reinterpret_cast<uint4*>(grp + static_cast<uint32_t>(pr * p.H * 16) + 8 * half) = uint4{s0[0], s1[0], s0[1], s1[1]};
-        }
+      for (int pr = 0; pr < 2; ++pr) {
+        const auto s0 = __builtin_amdgcn_permlane32_swap(w[4 * pr], w[4 * pr + 2], false, false);
+        const auto s1 = __builtin_amdgcn_permlane32_swap(w[4 * pr + 1], w[4 * pr + 3], false, false);
+        *reinterpret_cast<uint4*>(grp + static_cast<uint32_t>(pr * p.H * 16) + 8 * half) = uint4{s0[0], s1[0], s0[1], s1[1]};
       }
     }
-    if (lse_lane) {
+    if (half == 0) {
       float* ml = p.part_ml + (row * p.split_stride + split) * p.H * 2 + static_cast<uint32_t>(head * 2);
       ml[0] = m_run;
       ml[1] = l_run;
@@ -918,7 +912,7 @@ __global__ void __launch_bounds__(HG * 64) sparse_mqa_kernel(const AttnParams p)
   }
 
   if (!head_ok) return;
-  write_result<D, NOPE, NB>(p, rp.row, rp.b, rp.split, head, half, half == 0, 0, NB, m_run, l_run, acc_o);
+  write_result<D, NOPE>(p, rp.row, rp.b, rp.split, head, half, m_run, l_run, acc_o);
 }
 
 #include "attention_latent.h"
@@ -1021,7 +1015,8 @@ int dispatch_heads(const AttnParams& p_in, int64_t rows, hipStream_t s, bool* me
   if constexpr (D > 256) {
     static_assert(D == LatentSmem::D && LatentSmem::LDS <= 160 * 1024, "the latent kernel's shape and LDS budget");
     auto kern = sparse_mqa_latent_kernel<FMT, NOPE, false>;
-    auto kern_sel = sparse_mqa_latent_kernel<FMT, NOPE, true>;
+    auto kern_sel = kern;  // (mzk_sparse_mqa_select selects in the launch for FP8 entries only)
+    if constexpr (FMT == kFmtFp8) kern_sel = sparse_mqa_latent_kernel<FMT, NOPE, true>;
     // the dynamic-LDS limit is a per-device function attribute: set once per device
     static std::atomic<bool> attr_set[kMaxDevices] = {};  // setting it twice is harmless
     int dev = 0;
