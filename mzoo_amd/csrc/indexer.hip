@@ -878,7 +878,7 @@ __global__ void __launch_bounds__(kWaves * 64) indexer_scores_kernel(const IdxPa
 // 73 us, about 23 of them the query's and the scores' memory traffic and the rest within
 // 1.2 times of the head sums alone.  (The earlier form kept 4 key tiles in registers and
 // re-read every row's fragments and weights from LDS between drained pipelines: matrix unit
-// busy 32 % and vector unit 44 % of the time.)  1021 rows of 32 heads on 4004 MXFP4 keys,
+// busy 28 % and vector unit 39 % of the time; now 45 % and 58 %.)  1021 rows of 32 heads on 4004 MXFP4 keys,
 // which the row form served before: 35 -> 18.8 us.  Taken back: pinning one MFMA to 16 vector
 // operations (2 % slower), storing the -inf of the unseen keys from inside the loop (5 %
 // slower), 3 or 4 workgroups per compute unit's worth of key splits (up to 20 % slower where
