@@ -761,13 +761,15 @@ __device__ __forceinline__ void merge_in_launch(const AttnParams& p, int64_t row
   }
   __syncthreads();
   if (m_go) {
-    // an item = 8 * NP channels of a head.  At 4 and 16 splits NP leaves the slice 144 items, one
-    // pass of the 256 threads (288, two passes: 4 splits of 32 rows 30.0 -> 28.8 us the launch, 16
-    // of 8 rows 27.4 -> 25.7); at 2 and 8 splits fewer, wider items took as long or longer (2
-    // splits at NP 8, 64 rows 38.7 -> 39.5; 8 splits at NP 4, 16 rows 29.1 -> 29.3)
+    // an item = 8 * NP channels of a head.  At 16 splits NP leaves the slice 144 items, one pass of
+    // the 256 threads (288, two passes: 8 rows 27.4 -> 25.7 us the launch).  2, 4 and 8 splits stay
+    // at 2 or 3 passes: wider items took as long or longer at 2 and 8 (2 splits at NP 8, 64 rows
+    // 38.7 -> 39.5; 8 splits at NP 4, 16 rows 29.1 -> 29.3), and NP 8 at 4 splits beside them (30.0
+    // -> 28.8) left the kernel two spilled registers, whose scratch memory costs every launch
+    // 0.6 us (100 rows x 32 heads 16.2 -> 16.8)
     switch (p.nsplit) {
-      case 2: merge_slice<D, NOPE, NT, 4>(p, row, h0, split, tid); break;
-      case 4: merge_slice<D, NOPE, NT, 8>(p, row, h0, split, tid); break;
+      case 2:
+      case 4: merge_slice<D, NOPE, NT, 4>(p, row, h0, split, tid); break;
       case 8:
       case 16: merge_slice<D, NOPE, NT, 2>(p, row, h0, split, tid); break;
       default: merge_slice<D, NOPE, NT, 1>(p, row, h0, split, tid); break;
@@ -1099,7 +1101,7 @@ int combine_impl(const float* workspace, int64_t B, int64_t S, int H, int D, int
 // mode: the path a group spread over several XCDs takes).  The in-launch merge is exact but
 // not faster on MI355X: its tail (the arrival, then each split's reads of its siblings'
 // partials) costs what the merge launch does (both launches -> one, 128 heads: 2 splits of 64
-// rows 39.2 -> 38.7 us, 4 of 32 rows 27.8 -> 28.8, 8 of 16 rows 27.2 -> 29.1, 16 of 8 rows 22.7
+// rows 39.2 -> 38.7 us, 4 of 32 rows 27.9 -> 30.0, 8 of 16 rows 27.2 -> 29.1, 16 of 8 rows 22.7
 // -> 25.7, 32 of 4 rows 27.6 -> 29.7), and most where the splits of a group finish several
 // microseconds apart.
 std::atomic<int> g_merge_mode{0};
