@@ -761,16 +761,15 @@ __device__ __forceinline__ void merge_in_launch(const AttnParams& p, int64_t row
   }
   __syncthreads();
   if (m_go) {
-    // an item = 8 * NP channels of a head.  At 16 splits NP leaves the slice 144 items, one pass of
-    // the 256 threads (288, two passes: 8 rows 27.4 -> 25.7 us the launch).  2, 4 and 8 splits stay
-    // at 2 or 3 passes: wider items took as long or longer at 2 and 8 (2 splits at NP 8, 64 rows
-    // 38.7 -> 39.5; 8 splits at NP 4, 16 rows 29.1 -> 29.3), and NP 8 at 4 splits beside them (30.0
-    // -> 28.8) left the kernel two spilled registers, whose scratch memory costs every launch
-    // 0.6 us (100 rows x 32 heads 16.2 -> 16.8)
+    // an item = 8 * NP channels of a head.  At 8 and 16 splits NP leaves the slice 144 items, one
+    // pass of the 256 threads (288, two passes: 16 rows of 8 splits 30.4 -> 29.5 us the launch, 8 rows
+    // of 16 27.4 -> 25.7).  2 and 4 splits stay at 3 and 2 passes: NP 8 took 64 rows of 2 splits
+    // from 38.7 to 39.5, and at 4 splits alone (32 rows 30.0 -> 28.8) it left the kernel two spilled
+    // registers, whose scratch memory costs every launch 0.6 us (100 rows x 32 heads 16.2 -> 16.8)
     switch (p.nsplit) {
       case 2:
-      case 4: merge_slice<D, NOPE, NT, 4>(p, row, h0, split, tid); break;
-      case 8:
+      case 4:
+      case 8: merge_slice<D, NOPE, NT, 4>(p, row, h0, split, tid); break;
       case 16: merge_slice<D, NOPE, NT, 2>(p, row, h0, split, tid); break;
       default: merge_slice<D, NOPE, NT, 1>(p, row, h0, split, tid); break;
     }
@@ -1101,8 +1100,8 @@ int combine_impl(const float* workspace, int64_t B, int64_t S, int H, int D, int
 // mode: the path a group spread over several XCDs takes).  The in-launch merge is exact but
 // not faster on MI355X: its tail (the arrival, then each split's reads of its siblings'
 // partials) costs what the merge launch does (both launches -> one, 128 heads: 2 splits of 64
-// rows 39.2 -> 38.7 us, 4 of 32 rows 27.9 -> 30.0, 8 of 16 rows 27.2 -> 29.1, 16 of 8 rows 22.7
-// -> 25.7, 32 of 4 rows 27.6 -> 29.7), and most where the splits of a group finish several
+// rows 39.2 -> 38.7 us, 4 of 32 rows 27.9 -> 30.1, 8 of 16 rows 27.3 -> 29.5, 16 of 8 rows 22.8
+// -> 25.9, 32 of 4 rows 27.8 -> 29.7), and most where the splits of a group finish several
 // microseconds apart.
 std::atomic<int> g_merge_mode{0};
 
