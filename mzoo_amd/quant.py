@@ -60,12 +60,8 @@ def _fake_quant_fp4_block(x: torch.Tensor, block_size: int, e4m3_scales: bool = 
     return y.view(x.shape)
 
 
-def _take_out(out, want) -> tuple[torch.Tensor, torch.Tensor]:
-    """``out`` as the contiguous tensors of the wanted (shape, dtype) pairs on one device, or
-    new ones."""
-    (device, *specs) = want
-    if out is None:
-        return tuple(torch.empty(shape, dtype=dt, device=device) for shape, dt in specs)
+def _check_out(out, device, specs) -> tuple[torch.Tensor, torch.Tensor]:
+    """``out``, if it is contiguous tensors of the (shape, dtype) pairs on the device."""
     for t, (shape, dt) in zip(out, specs):
         if tuple(t.shape) != tuple(shape) or t.dtype != dt or t.device != device or not t.is_contiguous():
             raise ValueError(f"out: contiguous {dt} {tuple(shape)} on {device} expected, got {t.dtype} {tuple(t.shape)}")
@@ -80,8 +76,12 @@ def quant_fp8_block(x: torch.Tensor, block_size: int = 128, out=None) -> tuple[t
     if n % block_size:
         raise ValueError(f"quant_fp8_block: n={n} is not a multiple of block_size={block_size}")
     xc = x.contiguous()
-    codes, scales = _take_out(out, (x.device, (x.shape, torch.uint8),
-                                    ((*x.shape[:-1], n // block_size), torch.float32)))
+    groups = (*x.shape[:-1], n // block_size)
+    if out is None:
+        codes = torch.empty(x.shape, dtype=torch.uint8, device=x.device)
+        scales = torch.empty(groups, dtype=torch.float32, device=x.device)
+    else:
+        codes, scales = _check_out(out, x.device, ((x.shape, torch.uint8), (groups, torch.float32)))
     _lib.call("mzk_quant_fp8_block", xc.data_ptr(), _lib.dtype_code(x.dtype), _rows(xc), n, block_size,
               codes.data_ptr(), scales.data_ptr(), _lib.stream_of(x))
     return codes, scales
@@ -106,8 +106,12 @@ def quant_mxfp4(x: torch.Tensor, out=None) -> tuple[torch.Tensor, torch.Tensor]:
     if n % 32:
         raise ValueError(f"quant_mxfp4: n={n} is not a multiple of 32")
     xc = x.contiguous()
-    packed, e8m0 = _take_out(out, (x.device, ((*x.shape[:-1], n // 2), torch.uint8),
-                                   ((*x.shape[:-1], n // 32), torch.uint8)))
+    halves, blocks = (*x.shape[:-1], n // 2), (*x.shape[:-1], n // 32)
+    if out is None:
+        packed = torch.empty(halves, dtype=torch.uint8, device=x.device)
+        e8m0 = torch.empty(blocks, dtype=torch.uint8, device=x.device)
+    else:
+        packed, e8m0 = _check_out(out, x.device, ((halves, torch.uint8), (blocks, torch.uint8)))
     _lib.call("mzk_quant_mxfp4", xc.data_ptr(), _lib.dtype_code(x.dtype), _rows(xc), n, packed.data_ptr(),
               e8m0.data_ptr(), _lib.stream_of(x))
     return packed, e8m0
