@@ -59,6 +59,12 @@ __device__ __forceinline__ int lat_swz(int e) { return e & 7; }
 constexpr float kRoomNear = kLazy, kRoomAbove = 100.0f;    // log2 units above the reference
 constexpr float kMasked = -3.0e38f;                        // a masked entry's score: weight 0
 
+// Rows of more scores than this are loaded in whole lines and passed on through LDS.  A thread's own 32
+// scores are a line of their own, so loaded directly each instruction touches 64 lines: 8192 keys, one
+// row x 64 heads 22.0 -> 21.7 us the launch and its merge, 64 rows 28.4 -> 27.9; at 4096 keys
+// both take as long, at 512 LDS costs 0.15 us.
+constexpr int kStageScores = 4096;
+
 // A tile in flight: one thread's pieces of entry tid / 8.
 template <int FMT>
 struct LatRaw {
@@ -101,7 +107,7 @@ sparse_mqa_latent_kernel(const AttnParams p) {
     const int G4 = static_cast<int>(p.G) - 4;
 #pragma unroll
     for (int m = 0; m < SKPT / 4; ++m) {
-      const int o = SKPT * tid + 4 * m;
+      const int o = p.G > kStageScores ? 4 * (NT * m + tid) : SKPT * tid + 4 * m;
       sc4[m] = *reinterpret_cast<const float4*>(srow + (o <= G4 ? o : G4));
     }
   } else {
@@ -161,9 +167,23 @@ sparse_mqa_latent_kernel(const AttnParams p) {
     const RowSelLds lds{h1, h2, h3, sw, sw + 8, sw + 12};
     const int G = static_cast<int>(p.G), k = p.topk;
     const bool search = G > k;
-    if (search) {
-      row_sel_clear<NT>(lds, tid);
-      lds_barrier();
+    // A long row's scores come in whole lines and reach their thread, 32 neighbours each, through
+    // LDS: piece j of thread t's at slot j ^ (t / 2 & 7), so that both passes meet every bank once.
+    const bool staged = p.G > kStageScores;  // uniform
+    float4* const stage = reinterpret_cast<float4*>(smem + M::PB - 4 * 8192);
+    static_assert(4 * 8 * NT + (kHist1<NT> + kBins + kBins / 2 + 16) * 4 <= M::PB - 4 * 8192, "behind the selection's LDS");
+    if (staged) {
+#pragma unroll
+      for (int m = 0; m < SKPT / 4; ++m) {
+        const int t = (NT / 8) * m + (tid >> 3);
+        stage[8 * t + ((tid & 7) ^ ((t >> 1) & 7))] = sc4[m];
+      }
+    }
+    if (search) row_sel_clear<NT>(lds, tid);
+    if (search || staged) lds_barrier();
+    if (staged) {
+#pragma unroll
+      for (int m = 0; m < SKPT / 4; ++m) sc4[m] = stage[8 * tid + (m ^ ((tid >> 1) & 7))];
     }
     const int i0 = SKPT * tid;
     uint32_t key[SKPT];

@@ -164,7 +164,8 @@ def _spread(kind, b, g, gen):
 
 
 @pytest.mark.parametrize("kind", ["octaves", "one bin", "low bits", "few", "equal"])
-@pytest.mark.parametrize("g,topk", [(4, 4), (260, 128), (2048, 512), (2052, 512), (8192, 2048), (8192, 4), (8188, 1000)])
+@pytest.mark.parametrize("g,topk", [(4, 4), (260, 128), (2048, 512), (2052, 512), (8192, 2048), (8192, 4), (8188, 1000),
+                                    (4096, 1000), (4100, 1000)])
 def test_selected_list_at_every_level(dev, kind, g, topk):
     """The selection of 256 threads (the attention's own, and the top-k launch up to 2048 keys)
     against the oracle, with -inf entries between."""
