@@ -17,7 +17,7 @@
 // of D read K and V twice as often and exchanged partial scores: about 2100 cycles of LDS.
 // Measured, against that kernel: a causal prompt of 8192 rows x 128 heads, top-2048 of 2048
 // entries, 4.14 -> 2.94 ms (671 -> 947 TFLOP/s; a bf16 product of 16384^3 reaches 1360 on the
-// same card); the decode step of 32 rows over 8192 keys 68.9 -> 62.5 us.  A tile takes about
+// same card); the decode step of 32 rows over 8192 keys 68.4 -> 61.5 us.  A tile takes about
 // 2050 cycles (bf16; fp8 2280): one wave per SIMD issues an instruction every 5 cycles or so,
 // 250 of them a tile, and the barrier adds 180; deeper operand prefetch changed nothing.
 //
